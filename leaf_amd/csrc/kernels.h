@@ -120,14 +120,13 @@ void launch_gemm_w8a8_mfma(const int8_t* W, const float* w_scales, const float* 
                            const float* xs, int M, int N, int K, float* y, int epilogue, int32_t* acc_out,
                            const GemmTiles& tiles, int32_t* partial, hipStream_t stream);
 
+// FP32-math GEMM on the bf16 matrix cores (gemm_f32.hip): K % 4 == 0, 16-byte
+// aligned input and weights, quantized groups % 4 == 0.
+bool gemm_f32_supported(const WeightView& w, const float* x);
+void launch_gemm_f32(const WeightView& w, const float* x, int tokens, float* y, int epilogue, hipStream_t stream);
+
 // Returns the path used (1 GEMV, 2 generic, 3 GEMM) or a negative value when
 // the call cannot run (missing scratch for the GEMM quantization).
-// FP32-math prefill GEMM on f32 MFMA with LDS-staged tiles (gemm_f32.hip):
-// K % 32 == 0, 16-byte aligned input and weights, quantized groups % 16 == 0.
-bool gemm_f32_lds_supported(const WeightView& w, const float* x);
-void launch_gemm_f32_lds(const WeightView& w, const float* x, int tokens, float* y, int epilogue,
-                         hipStream_t stream);
-
 int launch_linear(const LinearCall& call, hipStream_t stream);
 // True when launch_linear runs the single-token integer GEMV that normalizes,
 // quantizes and applies paired epilogues inside the kernel.

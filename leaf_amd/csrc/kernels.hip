@@ -1054,87 +1054,6 @@ __global__ __launch_bounds__(kBlock) void gemm_w8a8_split_epilogue4(WeightView w
     }
 }
 
-// ------------------------------------------------ FP prefill: f32 MFMA ---
-// Y[t, n] = sum_k X[t, k] W[n, k] with v_mfma_f32_16x16x4_f32; weights of any
-// storage are widened (BF16) or dequantized (INT8 / INT4) as they are loaded.
-// Each lane loads four consecutive K values of its row and column and feeds
-// them to four MFMAs, so operand K positions always agree between A and B.
-template <int BITS>
-__device__ __forceinline__ float4 load_w4(const WeightView& w, int n, int k) {
-    // four consecutive values W[n, k..k+3], k a multiple of 4
-    if constexpr (BITS == 32) {
-        return *(const float4*)((const float*)w.data + (size_t)n * w.cols + k);
-    } else if constexpr (BITS == 16) {
-        const uint2 v = *(const uint2*)((const uint16_t*)w.data + (size_t)n * w.cols + k);
-        return make_float4(bf16_to_f32(v.x & 0xFFFFu), bf16_to_f32(v.x >> 16), bf16_to_f32(v.y & 0xFFFFu),
-                           bf16_to_f32(v.y >> 16));
-    } else {
-        float f[4];
-        const int groups = w.cols / w.group;
-        if constexpr (BITS == 8) {
-            const uint32_t v = *(const uint32_t*)((const int8_t*)w.data + (size_t)n * w.cols + k);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) f[e] = (float)(int)(int8_t)((v >> (8 * e)) & 0xFFu);
-        } else {
-            const uint16_t v = *(const uint16_t*)((const uint8_t*)w.data + ((size_t)n * w.cols + k) / 2);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) f[e] = (float)nibble((v >> (8 * (e / 2))) & 0xFFu, e & 1);
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) f[e] = f[e] * w.scales[(size_t)n * groups + (k + e) / w.group];
-        return make_float4(f[0], f[1], f[2], f[3]);
-    }
-}
-
-template <int BITS>
-__global__ __launch_bounds__(kBlock) void gemm_f32_kernel(WeightView w, const float* __restrict__ x, int tokens,
-                                                         float* __restrict__ y, int epilogue) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int K = w.cols, N = w.rows;
-    const int tile_m = blockIdx.y * 64 + (wave >> 1) * 32;
-    const int tile_n = blockIdx.x * 64 + (wave & 1) * 32;
-    const int li = lane & 15, lk = (lane >> 4) * 4;
-    v4f acc[2][2];
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = v4f{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < K; k0 += 16) {
-        const int k = k0 + lk;
-        float4 av[2], bv[2];
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-            const int t = tile_m + a * 16 + li;
-            av[a] = (t < tokens && k < K) ? *(const float4*)(x + (size_t)t * K + k) : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            const int n = tile_n + b * 16 + li;
-            bv[b] = (n < N && k < K) ? load_w4<BITS>(w, n, k) : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[a].x, bv[b].x, acc[a][b], 0, 0, 0);
-                acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[a].y, bv[b].y, acc[a][b], 0, 0, 0);
-                acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[a].z, bv[b].z, acc[a][b], 0, 0, 0);
-                acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[a].w, bv[b].w, acc[a][b], 0, 0, 0);
-            }
-    }
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            const int n = tile_n + b * 16 + li;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int t = tile_m + a * 16 + (lane >> 4) * 4 + i;
-                if (t < tokens && n < N) store_out(y, (size_t)t * N + n, acc[a][b][i], bias_at(w, n), epilogue);
-            }
-        }
-}
-
 // --------------------------------------------------------- RoPE + KV ---
 // rotary() + KV append (decoder.cpp:1259-1281, 1332-1343): head-major reorder,
 // rotate-half of the first `rotary` values with host-built cos/sin tables,
@@ -2184,18 +2103,8 @@ int launch_linear(const LinearCall& call, hipStream_t stream) {
         }
         return 1;
     }
-    if (path == 3 && !c.force_path && gemm_f32_lds_supported(w, c.x)) {
-        launch_gemm_f32_lds(w, c.x, c.tokens, c.y, c.epilogue, stream);
-        return 3;
-    }
-    if (path == 3) {
-        dim3 grid(ceil_div(w.rows, 64), ceil_div(c.tokens, 64));
-        switch (w.bits) {
-        case 32: gemm_f32_kernel<32><<<grid, kBlock, 0, stream>>>(w, c.x, c.tokens, c.y, c.epilogue); break;
-        case 16: gemm_f32_kernel<16><<<grid, kBlock, 0, stream>>>(w, c.x, c.tokens, c.y, c.epilogue); break;
-        case 8: gemm_f32_kernel<8><<<grid, kBlock, 0, stream>>>(w, c.x, c.tokens, c.y, c.epilogue); break;
-        default: gemm_f32_kernel<4><<<grid, kBlock, 0, stream>>>(w, c.x, c.tokens, c.y, c.epilogue); break;
-        }
+    if (path == 3 && gemm_f32_supported(w, c.x)) {
+        launch_gemm_f32(w, c.x, c.tokens, c.y, c.epilogue, stream);
         return 3;
     }
     linear_generic_kernel<<<ceil_div((size_t)c.tokens * w.rows, kBlock), kBlock, 0, stream>>>(

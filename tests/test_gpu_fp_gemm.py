@@ -1,0 +1,103 @@
+"""FP32-math linears of five and more tokens: the bf16-split GEMM (gemm_f32.hip).
+
+Every output is compared with its 64-bit value under the bound of a plain f32
+dot of K terms, K 2^-24 sum|x w| (the split GEMM rounds less often: once per
+MFMA product of 32 terms), plus 2^-24 sum|x w| for the products it leaves out
+and one rounding for the bias.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from leaf_amd.artifact import quantize
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def rt():
+    from leaf_amd import runtime
+    runtime.library()
+    return runtime
+
+
+def weights(rng, bits, N, K, group):
+    """(storage, scales, group, the weights in 64 bits)"""
+    w = (0.02 * rng.standard_normal((N, K))).astype(np.float32)
+    if bits == 32:
+        return w, None, 0, w.astype(np.float64)
+    if bits == 16:
+        data = (w.view(np.uint32) >> 16).astype(np.uint16)
+        return data, None, 0, (data.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    data, scales = quantize(w, bits, group)
+    q = data
+    if bits == 4:
+        q = np.empty((N, K), np.int8)
+        q[:, ::2], q[:, 1::2] = data & 15, data >> 4
+        q[q >= 8] -= 16
+    return data, scales, group, q.astype(np.float64) * np.repeat(scales.astype(np.float64), group, axis=1)
+
+
+def run(rt, bits, data, scales, group, bias, x):
+    dw = rt.DeviceWeight(data, bits, x.shape[1], scales, group, bias)
+    dx, dy = rt.DeviceArray.of(x), rt.DeviceArray((x.shape[0], data.shape[0]), np.float32)
+    rt.linear(dw, dx, x.shape[0], 32, dy)
+    return dy.numpy()
+
+
+def within_bound(y, x, wd, bias):
+    e = x.astype(np.float64) @ wd.T
+    size = np.abs(x).astype(np.float64) @ np.abs(wd).T
+    bound = (x.shape[1] + 1) * 2.0 ** -24 * size + 2.0 ** -23 * (np.abs(e) + np.abs(bias))
+    return bool(np.all(np.abs(y - (e + bias)) <= bound))
+
+
+# Token and row counts at the edges of the blocks (16 to 128 of either), grids
+# that choose each of them, K of one stage and odd counts of stages.
+@pytest.mark.parametrize("bits,group", [(32, 0), (16, 0), (8, 0), (8, 64), (4, 32)])
+@pytest.mark.parametrize("M,K,N", [(5, 64, 1), (16, 1984, 130), (33, 448, 777), (65, 64, 2051), (129, 960, 515),
+                                   (300, 4864, 96), (513, 192, 1030), (700, 896, 2100), (1100, 64, 33)])
+def test_shapes(rt, bits, group, M, K, N):
+    rng = np.random.default_rng(M + K + N + bits)
+    data, scales, group, wd = weights(rng, bits, N, K, group or K)
+    bias = (0.1 * rng.standard_normal(N)).astype(np.float32)
+    x = rng.standard_normal((M, K), dtype=np.float32)
+    x[rng.random((M, K)) < 0.001] *= np.float32(20)
+    assert within_bound(run(rt, bits, data, scales, group, bias, x), x, wd, bias)
+
+
+# Rows that end inside a 32-value stage, and scale groups that are not whole stages.
+@pytest.mark.parametrize("bits,K,group", [(32, 36, 0), (32, 772, 0), (16, 100, 0), (16, 1028, 0), (8, 100, 100),
+                                          (8, 96, 4), (8, 432, 48), (4, 100, 20), (4, 144, 16), (4, 1200, 100)])
+@pytest.mark.parametrize("M,N", [(7, 17), (77, 131), (400, 1000)])
+def test_ragged_rows_and_groups(rt, bits, K, group, M, N):
+    rng = np.random.default_rng(K + M)
+    data, scales, group, wd = weights(rng, bits, N, K, group)
+    bias = (0.1 * rng.standard_normal(N)).astype(np.float32)
+    x = rng.standard_normal((M, K), dtype=np.float32)
+    assert within_bound(run(rt, bits, data, scales, group, bias, x), x, wd, bias)
+
+
+@pytest.mark.parametrize("bits,K", [(32, 256), (16, 256), (8, 256), (4, 256), (32, 260)])
+@pytest.mark.parametrize("M,N", [(6, 40), (200, 1030)])
+def test_values_that_do_not_split(rt, bits, K, M, N):
+    # Infinities, NaN and values that round past bf16's largest: what a chain
+    # of f32 multiply-adds gives, in the outputs they reach and no other.
+    rng = np.random.default_rng(5 + bits)
+    data, scales, group, wd = weights(rng, bits, N, K, 32 if bits == 4 else K)
+    x = rng.standard_normal((M, K), dtype=np.float32)
+    huge = np.finfo(np.float32).max
+    x[0, 3], x[1, 5], x[2, 7], x[3, 9] = np.inf, -np.inf, np.nan, huge
+    x[4, 1], x[4, 2] = np.inf, -np.inf
+    if bits == 32:
+        data[11, 20] = np.inf
+        wd = data.astype(np.float64)
+    y = run(rt, bits, data, scales, group, None, x)
+    with np.errstate(all="ignore"):
+        e = x.astype(np.float64) @ wd.T
+        e = np.where(np.abs(e) > huge, np.sign(e) * np.inf, e)
+        assert np.array_equal(np.isnan(y), np.isnan(e))
+        assert np.array_equal(np.isinf(y), np.isinf(e)) and np.array_equal(np.sign(y[np.isinf(y)]), np.sign(e[np.isinf(e)]))
+        plain = np.isfinite(e)
+        assert np.all(np.abs(y - e)[plain] <= 1e-4 * (1 + np.abs(e[plain])))
