@@ -120,6 +120,12 @@ void launch_gemm_w8a8_mfma(const int8_t* W, const float* w_scales, const float* 
                            const float* xs, int M, int N, int K, float* y, int epilogue, int32_t* acc_out,
                            const GemmTiles& tiles, int32_t* partial, hipStream_t stream);
 
+// Integer-activation GEMM for int8 / int4 weights with scale groups of whole
+// multiples of 32 values (gemm_grouped.hip), 16-byte aligned operands.
+bool gemm_grouped_supported(const WeightView& w, const int8_t* xq);
+void launch_gemm_grouped(const WeightView& w, const int8_t* xq, const float* xs, int tokens, float* y, int epilogue,
+                         int32_t* acc_out, bool unfused, hipStream_t stream);
+
 // FP32-math GEMM on the bf16 matrix cores (gemm_f32.hip): K % 4 == 0, 16-byte
 // aligned input and weights, quantized groups % 4 == 0.
 bool gemm_f32_supported(const WeightView& w, const float* x);

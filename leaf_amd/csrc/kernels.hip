@@ -926,87 +926,6 @@ __global__ __launch_bounds__(kBlock) void linear_generic_kernel(WeightView w, co
     store_out(y, (size_t)t * w.rows + row, result, bias_at(w, row), epilogue);
 }
 
-// ------------------------------------------------ W8A8 prefill: int8 MFMA ---
-// Y[t, n] = sum_k Xq[t, k] W[n, k] with v_mfma_i32_16x16x64_i8.  A 64x64 block
-// tile, four waves of 32x32 (2x2 MFMA tiles).  Lane l feeds row/column (l & 15)
-// with 16 consecutive K bytes at offset 16 * (l >> 4) of each 64-wide K step,
-// for both operands, so the exact integer sum does not depend on how the
-// hardware orders K inside the instruction.  Accumulators are exact; the
-// epilogue is the CPU path's per group (group_term).
-__global__ __launch_bounds__(kBlock) void gemm_int8_kernel(WeightView w, const int8_t* __restrict__ xq,
-                                                          const float* __restrict__ xs, int tokens,
-                                                          float* __restrict__ y, int epilogue,
-                                                          int32_t* __restrict__ acc_out, int unfused) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int K = w.cols, N = w.rows;
-    const int tile_m = blockIdx.y * 64 + (wave >> 1) * 32;   // tokens
-    const int tile_n = blockIdx.x * 64 + (wave & 1) * 32;    // weight rows
-    const int li = lane & 15, lk = (lane >> 4) * 16;
-    const int groups = K / w.group;
-    const int steps_per_group = w.group / 64;
-    v4i acc[2][2];
-    float res[2][2][4];
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            acc[a][b] = v4i{0, 0, 0, 0};
-#pragma unroll
-            for (int i = 0; i < 4; ++i) res[a][b][i] = 0.0f;
-        }
-    const int8_t* wbase = (const int8_t*)w.data;
-    const int steps = K / 64;
-    for (int s = 0; s < steps; ++s) {
-        const int k = s * 64 + lk;
-        v4i av[2], bv[2];
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-            const int t = tile_m + a * 16 + li;
-            av[a] = t < tokens ? *(const v4i*)(xq + (size_t)t * K + k) : v4i{0, 0, 0, 0};
-        }
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            const int n = tile_n + b * 16 + li;
-            bv[b] = n < N ? __builtin_nontemporal_load((const v4i*)(wbase + (size_t)n * K + k)) : v4i{0, 0, 0, 0};
-        }
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int b = 0; b < 2; ++b)
-                acc[a][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[a], bv[b], acc[a][b], 0, 0, 0);
-        if ((s + 1) % steps_per_group == 0) {
-            const int g = (s + 1) / steps_per_group - 1;
-#pragma unroll
-            for (int a = 0; a < 2; ++a)
-#pragma unroll
-                for (int b = 0; b < 2; ++b) {
-                    const int n = tile_n + b * 16 + li;
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const int t = tile_m + a * 16 + (lane >> 4) * 4 + i;
-                        if (t < tokens && n < N) {
-                            if (acc_out) acc_out[((size_t)t * N + n) * groups + g] = acc[a][b][i];
-                            res[a][b][i] = group_term(acc[a][b][i], xs[t], w.scales[(size_t)n * groups + g],
-                                                      res[a][b][i], unfused);
-                        }
-                    }
-                    acc[a][b] = v4i{0, 0, 0, 0};
-                }
-        }
-    }
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            const int n = tile_n + b * 16 + li;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int t = tile_m + a * 16 + (lane >> 4) * 4 + i;
-                if (t < tokens && n < N) store_out(y, (size_t)t * N + n, res[a][b][i], bias_at(w, n), epilogue);
-            }
-        }
-}
-
 // ---------------------- W8A8 prefill, per-row scales: split-K epilogue ---
 // The MFMA GEMM (gemm_w8a8.hip) stores each K split's exact int32 sums to
 // partial[split][t][n]; this adds them in split order and applies the CPU
@@ -2024,9 +1943,12 @@ int launch_linear(const LinearCall& call, hipStream_t stream) {
         const bool per_row = w.group == K;
         const bool fast = per_row && chunked;
         int path = c.force_path;
-        if (!path) path = (fast && c.tokens <= 4) ? 1 : (w.bits == 8 && c.tokens > 4 && K % 64 == 0 && w.group % 64 == 0) ? 3 : 2;
+        // the input as the GEMMs will see it: given, or quantized into the scratch
+        const bool gemm = (per_row && w.bits == 8 && gemm_w8a8_mfma_supported(K) && aligned(w.data)) ||
+                          gemm_grouped_supported(w, c.xq ? c.xq : c.xq_scratch);
+        if (!path) path = (fast && c.tokens <= 4) ? 1 : gemm && (c.tokens > 4 || !per_row) ? 3 : 2;
         if (path == 1 && !(fast && c.tokens <= 4)) path = 2;
-        if (path == 3 && !(w.bits == 8 && K % 64 == 0 && w.group % 64 == 0 && aligned(w.data))) path = 2;
+        if (path == 3 && !gemm) path = 2;
         const int E8 = w.bits == 8 ? 16 : 32;
         if (path == 1 && c.tokens == 1 && c.x && !c.xq && K <= kFusedMaxK) {
             if (w.bits == 8) launch_fused_int<8>(c, stream); else launch_fused_int<4>(c, stream);
@@ -2046,7 +1968,7 @@ int launch_linear(const LinearCall& call, hipStream_t stream) {
             if (w.bits == 8) launch_gemv_int<8>(c, xq, xs, stream); else launch_gemv_int<4>(c, xq, xs, stream);
             return 1;
         }
-        if (path == 3 && w.group == K && gemm_w8a8_mfma_supported(K)) {
+        if (path == 3 && per_row && w.bits == 8 && gemm_w8a8_mfma_supported(K)) {
             const GemmTiles tiles = gemm_w8a8_tiles(c.tokens, w.rows, K, c.split_scratch ? c.split_capacity : 0);
             int32_t* partial = tiles.splits > 1 ? c.split_scratch : nullptr;
             const int splits = tiles.splits;
@@ -2068,9 +1990,8 @@ int launch_linear(const LinearCall& call, hipStream_t stream) {
             return 3;
         }
         if (path == 3) {
-            dim3 grid(ceil_div(w.rows, 64), ceil_div(c.tokens, 64));
-            gemm_int8_kernel<<<grid, kBlock, 0, stream>>>(w, xq, xs, c.tokens, c.y, c.epilogue, c.acc_out,
-                                                          c.unfused_group_sum && c.tokens > 1);
+            launch_gemm_grouped(w, xq, xs, c.tokens, c.y, c.epilogue, c.acc_out, c.unfused_group_sum && c.tokens > 1,
+                                stream);
             return 3;
         }
         linear_generic_kernel<<<ceil_div((size_t)c.tokens * w.rows, kBlock), kBlock, 0, stream>>>(
