@@ -124,6 +124,17 @@ void* scratch_bytes(size_t bytes, hipStream_t stream) {
     return sc.work->ptr;
 }
 
+// scratch_bytes for work that can also run without: null where the stream is
+// capturing and its scratch is too small.
+void* scratch_bytes_if_available(size_t bytes, hipStream_t stream) {
+    {
+        std::lock_guard<std::mutex> guard(g_scratch_lock);
+        StreamScratch& sc = scratch_of(stream);
+        if ((!sc.work || sc.work->bytes < bytes) && capturing(stream)) return nullptr;
+    }
+    return scratch_bytes(bytes, stream);
+}
+
 // Zero-initialized span counters of the decode attention kernel (it resets
 // them itself), one set per (device, stream).
 unsigned* attention_counters(hipStream_t stream) {
@@ -726,6 +737,11 @@ lh_status lh_attention(const float* q_heads, const float* keys, const float* val
             a.partial = static_cast<float*>(scratch_bytes(floats * sizeof(float), as_stream(stream)));
             a.partial_capacity = int(floats);
             a.counters = attention_counters(as_stream(stream));
+        } else if (tokens > 1 && leafhip::attention_rows_supported(a.dim)) {
+            const size_t floats = leafhip::attention_rows_scratch_floats(a);
+            if (floats && floats <= 0x7fffffff)
+                a.partial = static_cast<float*>(scratch_bytes_if_available(floats * sizeof(float), as_stream(stream)));
+            a.partial_capacity = a.partial ? int(floats) : 0;
         }
         leafhip::check(leafhip::launch_attention(a, as_stream(stream)), "attention launch rejected", LH_ERROR_UNSUPPORTED);
         leafhip::hip_check(hipGetLastError(), "attention launch");

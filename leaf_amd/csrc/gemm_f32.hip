@@ -30,12 +30,10 @@
 
 #include "device_common.h"
 #include "kernels.h"
+#include "split_bf16.h"
 
 namespace leafhip {
 namespace {
-
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 
 constexpr int kStageK = 32;    // K values per stage: one MFMA's
 
@@ -45,22 +43,6 @@ enum WeightMode : int {
     kExactGroup = 1,    // one plane of integers, a scale per group of whole stages
     kSplit = 2,         // f32, or any other grouping dequantized to f32: three planes
 };
-
-// x as three bf16 values, without loss.
-__device__ __forceinline__ void split8(const float (&f)[8], v8bf& hi, v8bf& mid, v8bf& lo) {
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        const v2f v = v2f{f[2 * p], f[2 * p + 1]};
-        const v2bf h = __builtin_convertvector(v, v2bf);
-        const v2f r = v2f{v.x - (float)h.x, v.y - (float)h.y};
-        const v2bf m = __builtin_convertvector(r, v2bf);
-        const v2f s = v2f{r.x - (float)m.x, r.y - (float)m.y};
-        const v2bf l = __builtin_convertvector(s, v2bf);
-        hi[2 * p] = h.x; hi[2 * p + 1] = h.y;
-        mid[2 * p] = m.x; mid[2 * p + 1] = m.y;
-        lo[2 * p] = l.x; lo[2 * p + 1] = l.y;
-    }
-}
 
 // Eight consecutive values of a weight row as stored.
 template <int BITS>

@@ -176,6 +176,14 @@ struct AttentionCall {
 // (position_ptr) is only supported by the single-token decode kernels.
 bool launch_attention(const AttentionCall& call, hipStream_t stream);
 
+// Attention of several tokens on the bf16 matrix cores (attention_prefill.hip),
+// head dims up to 128 in multiples of 4.
+bool attention_rows_supported(int dim);
+// Floats of `partial` with which a call splits its keys over blocks as it would
+// like to (0: not at all); with fewer it runs unsplit.
+size_t attention_rows_scratch_floats(const AttentionCall& call);
+void launch_attention_rows(const AttentionCall& call, hipStream_t stream);
+
 // act = up * activate(gate) for gated MLPs, act = activate(up) otherwise.
 // gate_up holds [tokens, 2 * width] = [gate | up] when gated, [tokens, width] otherwise.
 void launch_activation(const float* gate_up, int tokens, int width, int gated, int activation, float* act,

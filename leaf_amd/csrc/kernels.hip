@@ -1011,6 +1011,46 @@ __global__ void rope_kv_kernel(RopeKvCall p) {
     }
 }
 
+// The same four values a thread (every width and pointer a multiple of 16
+// bytes), no thread idle: a rotated quad with its partner, a copied quad of a
+// q or k head, or a quad of v.  2048 tokens x 18 heads of 64: 7.0 us (9.2 with
+// one value a thread).
+__global__ __launch_bounds__(kBlock) void rope_kv_quads_kernel(RopeKvCall p) {
+    const int t = blockIdx.y;
+    const int turned = p.rotary / 8, per_head = turned + (p.dim - p.rotary) / 4;
+    const int qk_items = (p.heads + p.kv_heads) * per_head;
+    const int item = blockIdx.x * blockDim.x + threadIdx.x;
+    if (item >= qk_items + p.kv_heads * (p.dim / 4)) return;
+    const float* row = p.qkv + (size_t)t * p.ld;
+    const int pos = (p.position_ptr ? *p.position_ptr : p.position) + t;
+    if (item >= qk_items) {
+        const int vh = (item - qk_items) / (p.dim / 4), i = (item - qk_items) % (p.dim / 4) * 4;
+        *(v4f*)(p.values + ((size_t)vh * p.capacity + pos) * p.dim + i) = *(const v4f*)(row + p.v_offset + vh * p.dim + i);
+        return;
+    }
+    const int hh = item / per_head, quad = item % per_head;
+    const float* src;
+    float* dst;
+    if (hh < p.heads) {
+        src = row + p.q_offset + hh * p.dim;
+        dst = p.q_heads + ((size_t)hh * p.tokens + t) * p.dim;
+    } else {
+        const int kh = hh - p.heads;
+        src = row + p.k_offset + kh * p.dim;
+        dst = p.keys + ((size_t)kh * p.capacity + pos) * p.dim;
+    }
+    if (quad < turned) {
+        const int half = p.rotary / 2, i = 4 * quad;
+        const v4f c = *(const v4f*)(p.cosines + (size_t)pos * half + i), s = *(const v4f*)(p.sines + (size_t)pos * half + i);
+        const v4f a = *(const v4f*)(src + i), b = *(const v4f*)(src + i + half);
+        *(v4f*)(dst + i) = a * c - b * s;
+        *(v4f*)(dst + i + half) = b * c + a * s;
+    } else {
+        const int i = p.rotary + 4 * (quad - turned);
+        *(v4f*)(dst + i) = *(const v4f*)(src + i);
+    }
+}
+
 // ------------------------------------------------------------ attention ---
 // Online-softmax GQA attention (kv head = h / (heads / kv_heads), by index;
 // transformer.cpp:94-146).  Scores use the CPU's sequential dot order and
@@ -1099,210 +1139,6 @@ __global__ __launch_bounds__(kBlock) void attention_kernel(AttentionCall p, int 
         for (int d = threadIdx.x; d < dim; d += blockDim.x)
             part[2 + d] = (o_s[0][d] + o_s[1][d]) + (o_s[2][d] + o_s[3][d]);
     }
-}
-
-// ----------------------------------------- prefill attention: f32 MFMA ---
-// Flash attention for head dim 64 (every supported decoder family).  A work
-// item is one query head and 32 tokens; waves w + 2 s (w < 2, s <
-// kPrefillSlices) own tokens t0 + 16w .. +15, wave w + 2 s the 16-key slices
-// s, s + kPrefillSlices, ... of each key tile, each with its own online
-// softmax; the states merge at the end (several waves per SIMD, so one's
-// MFMAs overlap another's softmax).  Items are numbered token-tile-major, and
-// block b runs item b, then item n - 1 - b: a causal prefill's short and long
-// key ranges pair up, so every block does about the same work.  Key
-// tiles of 64 keys are staged in LDS (K and V, rows padded to 68 floats: the
-// MFMA operand reads then hit every bank twice, the minimum for 64 lanes),
-// the next tile waiting in registers while this one is used.
-//
-// Per 16 keys a wave computes S^T = K Q^T with v_mfma_f32_16x16x4_f32 (lane l
-// feeds key row l % 16 and query column l % 16 at dims 4c + l / 16), which
-// leaves lane l with the scores of query l % 16 for keys 4 (l / 16) + r,
-// r < 4: exactly the B operand of O^T += V^T P^T when that product takes the
-// keys {4j + r} as its K dimension.  So P never leaves registers.  Softmax is
-// online per query (max and sum exchanged between the four lanes of a query),
-// scores are (q.k * scale) * scale and masked keys are -inf, as in
-// transformer.cpp:112-143; the output is divided by the sum at the end.
-constexpr int kPrefillQ = 32;        // tokens per work item
-constexpr int kPrefillGroups = kPrefillQ / 16;
-constexpr int kPrefillKeys = 64;     // keys per LDS tile
-constexpr int kPrefillStride = 68;   // padded row of a K or V tile
-constexpr int kPrefillSlices = 4;    // waves per 16-token group
-constexpr int kPrefillThreads = kPrefillGroups * kWave * kPrefillSlices;
-constexpr int kPrefillLoads = 1024 / kPrefillThreads;   // float4 of a 64 x 64 tile per thread
-constexpr int kPrefillMerge = 18;    // merge record per lane: O^T (16), max, sum
-constexpr int kPrefillLds = 2 * kPrefillKeys * kPrefillStride > (kPrefillSlices - 1) * kPrefillGroups * kWave * kPrefillMerge
-                                ? 2 * kPrefillKeys * kPrefillStride
-                                : (kPrefillSlices - 1) * kPrefillGroups * kWave * kPrefillMerge;
-
-// One thread's share of a 64 x 64 K (and V) tile: float4 i, i + kPrefillThreads, ...
-// Rows at or past `end` were never written (they may hold NaN, and a masked
-// key still multiplies its V row by 0): they load row 0 and are stored as
-// zeros.  (The loaded values are not touched until the store, so the loads
-// stay in flight while the current tile is used.)
-__device__ __forceinline__ void prefill_tile_load(const float* K, const float* V, int k0, int end,
-                                                  v4f (&kr)[kPrefillLoads], v4f (&vr)[kPrefillLoads]) {
-#pragma unroll
-    for (int j = 0; j < kPrefillLoads; ++j) {
-        const int f = threadIdx.x + kPrefillThreads * j, row = f / 16, col = 4 * (f % 16);
-        const int key = k0 + row;
-        const size_t at = (size_t)(key < end ? key : 0) * 64 + col;
-        kr[j] = *(const v4f*)(K + at);
-        vr[j] = *(const v4f*)(V + at);
-    }
-}
-__device__ __forceinline__ void prefill_tile_store(float* ks, float* vs, const v4f (&kr)[kPrefillLoads],
-                                                   const v4f (&vr)[kPrefillLoads], int k0, int end) {
-#pragma unroll
-    for (int j = 0; j < kPrefillLoads; ++j) {
-        const int f = threadIdx.x + kPrefillThreads * j, row = f / 16, col = 4 * (f % 16);
-        const bool ok = k0 + row < end;
-        const v4f zero = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-        *(v4f*)(ks + row * kPrefillStride + col) = ok ? kr[j] : zero;
-        *(v4f*)(vs + row * kPrefillStride + col) = ok ? vr[j] : zero;
-    }
-}
-
-// One work item: query head h, tokens t0 .. t0 + kPrefillQ - 1.  Starts and
-// ends with a barrier, so items can follow each other on the same LDS.
-__device__ __forceinline__ void attention_prefill_item(const AttentionCall& p, int h, int t0, float* lds) {
-    float* ks = lds;
-    float* vs = lds + kPrefillKeys * kPrefillStride;
-    constexpr int dim = 64;
-    constexpr int kMerge = kPrefillMerge;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int group = wave % kPrefillGroups, slice = wave / kPrefillGroups;   // token group, key slice
-    const int li = lane & 15, lj = lane >> 4;
-    const int kvh = h / (p.heads / p.kv_heads);
-    const int tw = t0 + 16 * group;                   // this wave's first token
-    const int q_tok = tw + li;                        // this lane's query (score columns)
-    const int q_pos = p.position + q_tok;
-    const bool q_live = q_tok < p.tokens;
-    // Q^T operand: dims 4c + lj of query q_tok
-    float qv[16];
-#pragma unroll
-    for (int c = 0; c < 16; ++c)
-        qv[c] = q_live ? p.q_heads[((size_t)h * p.tokens + q_tok) * dim + 4 * c + lj] : 0.0f;
-    // keys the block needs: [first, end)
-    const int last_tok = min(t0 + kPrefillQ, p.tokens) - 1;
-    const int end = p.position + last_tok + 1;
-    int first = 0;
-    if (p.window) first = max(0, p.position + t0 + 1 - p.window);
-    first &= ~(kPrefillKeys - 1);
-    const float* K = p.keys + (size_t)kvh * p.capacity * dim;
-    const float* V = p.values + (size_t)kvh * p.capacity * dim;
-    v4f kr[kPrefillLoads], vr[kPrefillLoads];
-    prefill_tile_load(K, V, first, end, kr, vr);
-    v4f o[4];   // O^T: dims 16 dc + 4 lj + i, query li
-#pragma unroll
-    for (int dc = 0; dc < 4; ++dc) o[dc] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-    float m = -INFINITY, l = 0.0f;
-    const float scale = p.scale;
-    for (int k0 = first; k0 < end; k0 += kPrefillKeys) {
-        lds_barrier();     // the previous tile is no longer read (the next one's loads stay in flight)
-        prefill_tile_store(ks, vs, kr, vr, k0, end);
-        lds_barrier();
-        if (k0 + kPrefillKeys < end) prefill_tile_load(K, V, k0 + kPrefillKeys, end, kr, vr);
-        // the keys this wave can see in this tile
-        const int wave_end = min(end, p.position + min(tw + 16, p.tokens));
-        for (int sub = 16 * slice; sub < kPrefillKeys && k0 + sub < wave_end; sub += 16 * kPrefillSlices) {
-            v4f sc = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-            const float* krow = ks + (sub + li) * kPrefillStride + lj;
-            float kv[16];   // all of the chain's K operands first: one LDS wait, not eight
-#pragma unroll
-            for (int c = 0; c < 16; ++c) kv[c] = krow[4 * c];
-            __builtin_amdgcn_sched_barrier(0);   // keep the reads batched ahead of the chain
-#pragma unroll
-            for (int c = 0; c < 16; ++c) sc = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[c], qv[c], sc, 0, 0, 0);
-            // the V operands of O^T += V^T P^T below, read while the softmax runs
-            float vv[4][4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-#pragma unroll
-                for (int dc = 0; dc < 4; ++dc) vv[r][dc] = vs[(sub + 4 * lj + r) * kPrefillStride + li + 16 * dc];
-            __builtin_amdgcn_sched_barrier(0);
-            // lane: query q_tok, keys k0 + sub + 4 lj + r
-            float e[4];
-            float tile_max = -INFINITY;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int key = k0 + sub + 4 * lj + r;
-                const bool ok = q_live && key <= q_pos && (p.window == 0 || key > q_pos - p.window);
-                e[r] = ok ? sc[r] * scale * scale : -INFINITY;
-                tile_max = fmaxf(tile_max, e[r]);
-            }
-            tile_max = max_xor16(tile_max);
-            tile_max = max_xor32(tile_max);
-            const float m_new = fmaxf(m, tile_max);
-            const float alpha = m_new == -INFINITY ? 1.0f : expf(m - m_new);
-            float tile_sum = 0.0f;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                e[r] = m_new == -INFINITY ? 0.0f : expf(e[r] - m_new);
-                tile_sum += e[r];
-            }
-            tile_sum = add_xor16(tile_sum);
-            tile_sum = add_xor32(tile_sum);
-            l = l * alpha + tile_sum;
-            m = m_new;
-#pragma unroll
-            for (int dc = 0; dc < 4; ++dc) o[dc] = o[dc] * alpha;
-            // O^T += V^T P^T over keys {4 j + r}: lane supplies V[4 lj + r][16 dc + li]
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-#pragma unroll
-                for (int dc = 0; dc < 4; ++dc)
-                    o[dc] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[r][dc], e[r], o[dc], 0, 0, 0);
-        }
-    }
-    // merge the other slices' states into slice 0's wave of the same tokens
-    __syncthreads();             // the last tile is no longer read
-    if (slice > 0) {
-        float* dst = lds + (((slice - 1) * kPrefillGroups + group) * kWave + lane) * kMerge;
-#pragma unroll
-        for (int dc = 0; dc < 4; ++dc)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) dst[4 * dc + i] = o[dc][i];
-        dst[16] = m;
-        dst[17] = l;
-    }
-    __syncthreads();
-    if (slice == 0) {
-        float mt = m;
-#pragma unroll
-        for (int z = 1; z < kPrefillSlices; ++z)
-            mt = fmaxf(mt, lds[(((z - 1) * kPrefillGroups + group) * kWave + lane) * kMerge + 16]);
-        const float a0 = m == -INFINITY ? 0.0f : expf(m - mt);
-        l = l * a0;
-#pragma unroll
-        for (int dc = 0; dc < 4; ++dc) o[dc] = o[dc] * a0;
-#pragma unroll
-        for (int z = 1; z < kPrefillSlices; ++z) {
-            const float* src = lds + (((z - 1) * kPrefillGroups + group) * kWave + lane) * kMerge;
-            const float a = src[16] == -INFINITY ? 0.0f : expf(src[16] - mt);
-            l = l + src[17] * a;
-#pragma unroll
-            for (int dc = 0; dc < 4; ++dc)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) o[dc][i] = o[dc][i] + src[4 * dc + i] * a;
-        }
-    }
-    if (slice == 0 && q_live) {
-        float* out = p.out + ((size_t)q_tok * p.heads + h) * dim;
-#pragma unroll
-        for (int dc = 0; dc < 4; ++dc) {
-            const v4f v = l > 0.0f ? v4f{o[dc][0] / l, o[dc][1] / l, o[dc][2] / l, o[dc][3] / l}
-                                   : v4f{0.0f, 0.0f, 0.0f, 0.0f};
-            *(v4f*)(out + 16 * dc + 4 * lj) = v;
-        }
-    }
-    __syncthreads();   // the merge records are read before the next item's tile lands
-}
-
-__global__ __launch_bounds__(kPrefillThreads) void attention_prefill_kernel(AttentionCall p, int items) {
-    __shared__ float lds[kPrefillLds];
-    const int first = blockIdx.x, second = items - 1 - (int)blockIdx.x;
-    attention_prefill_item(p, first % p.heads, (first / p.heads) * kPrefillQ, lds);
-    if (second > first) attention_prefill_item(p, second % p.heads, (second / p.heads) * kPrefillQ, lds);
 }
 
 __global__ void attention_merge_kernel(AttentionCall p, int splits) {
@@ -2034,6 +1870,17 @@ int launch_linear(const LinearCall& call, hipStream_t stream) {
 }
 
 void launch_rope_kv(const RopeKvCall& call, hipStream_t stream) {
+    auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    // (one token keeps the kernel of one value a thread: its few blocks' latency
+    // is what counts, and its threads do less each)
+    if (call.tokens > 1 && call.dim % 4 == 0 && call.rotary % 8 == 0 && call.ld % 4 == 0 && call.q_offset % 4 == 0 && call.k_offset % 4 == 0 &&
+        call.v_offset % 4 == 0 && aligned(call.qkv) && aligned(call.cosines) && aligned(call.sines) &&
+        aligned(call.q_heads) && aligned(call.keys) && aligned(call.values)) {
+        const int quads = (call.heads + call.kv_heads) * (call.rotary / 8 + (call.dim - call.rotary) / 4) +
+                          call.kv_heads * (call.dim / 4);
+        rope_kv_quads_kernel<<<dim3(ceil_div(quads, kBlock), call.tokens), kBlock, 0, stream>>>(call);
+        return;
+    }
     const int items = (call.heads + 2 * call.kv_heads) * call.dim;
     dim3 grid(ceil_div(items, kBlock), call.tokens);
     rope_kv_kernel<<<grid, kBlock, 0, stream>>>(call);
@@ -2071,9 +1918,8 @@ bool launch_attention(const AttentionCall& call, hipStream_t stream) {
         }
         if (splits == 1) per_split = total;
     }
-    if (splits == 1 && call.tokens > 1 && call.dim == 64) {
-        const int items = call.heads * ((call.tokens + kPrefillQ - 1) / kPrefillQ);
-        attention_prefill_kernel<<<(items + 1) / 2, kPrefillThreads, 0, stream>>>(call, items);
+    if (call.tokens > 1 && attention_rows_supported(call.dim)) {
+        launch_attention_rows(call, stream);
         return true;
     }
     dim3 grid(call.heads, call.tokens, splits);

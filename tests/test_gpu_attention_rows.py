@@ -1,0 +1,110 @@
+"""Attention of several tokens on the bf16 matrix cores (attention_prefill.hip) and the quad RoPE + append.
+
+Outputs against 64-bit attention: the scores and sums are f32 sums of exact
+products, so an output differs by a few units of 2^-24 of the largest value
+times the chain of roundings in a weight (scores of up to about 30 in size).
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def rt():
+    from leaf_amd import runtime
+    runtime.library()
+    return runtime
+
+
+def exact(q, keys, values, position, window):
+    heads, tokens, dim = q.shape
+    group = heads // keys.shape[0]
+    out = np.empty((tokens, heads, dim))
+    for h in range(heads):
+        k, v = (a[h // group].astype(np.float64) for a in (keys, values))
+        for t in range(tokens):
+            end = position + t + 1
+            begin = max(0, end - window) if window else 0
+            s = k[begin:end] @ q[h, t].astype(np.float64) / np.sqrt(dim)
+            p = np.exp(s - s.max())
+            out[t, h] = (p / p.sum()) @ v[begin:end]
+    return out
+
+
+def call(rt, q, keys, values, position, window):
+    heads, tokens, dim = q.shape
+    kv, capacity, _ = keys.shape
+    dq, dk, dv = (rt.DeviceArray.of(a) for a in (q, keys, values))
+    out = rt.DeviceArray((tokens, heads, dim), np.float32)
+    rt.check(rt.library().lh_attention(dq.ptr, dk.ptr, dv.ptr, capacity, heads, kv, dim, tokens, position, window,
+                                       out.ptr, None))
+    return out.numpy()
+
+
+def inputs(rng, tokens, position, heads, kv, dim):
+    total, capacity = position + tokens, position + tokens + 37
+    q = rng.standard_normal((heads, tokens, dim), dtype=np.float32)
+    keys, values = (rng.standard_normal((kv, capacity, dim), dtype=np.float32) for _ in range(2))
+    keys[:, total:] = values[:, total:] = np.nan      # never written
+    return q, keys, values
+
+
+# Row tiles (128 rows, 64 beyond 64 values) cut by the token count, groups that
+# do not divide them, one part and several (few rows over long caches), every
+# padded width, windows shorter and longer than a step of 64 keys.
+@pytest.mark.parametrize("tokens,position,heads,kv,dim,window", [
+    (2, 0, 12, 12, 64, 0), (2, 700, 14, 2, 64, 0), (3, 64, 7, 1, 32, 0), (17, 0, 15, 5, 64, 0), (33, 191, 4, 1, 128, 0),
+    (64, 0, 32, 4, 64, 0), (65, 1, 6, 2, 80, 0), (130, 40, 5, 5, 96, 0), (40, 0, 3, 3, 4, 0), (50, 90, 4, 2, 20, 33),
+    (90, 300, 6, 3, 64, 100), (70, 500, 8, 2, 128, 64), (5, 1500, 32, 8, 128, 0), (300, 20, 2, 1, 36, 7)])
+def test_against_64_bits(rt, tokens, position, heads, kv, dim, window):
+    rng = np.random.default_rng(tokens * 31 + position + dim)
+    q, keys, values = inputs(rng, tokens, position, heads, kv, dim)
+    got, want = call(rt, q, keys, values, position, window), exact(q, keys, values, position, window)
+    assert np.isfinite(got).all()
+    # weights to 2^-24 (|score| + 8), so outputs to that of the largest value
+    assert np.max(np.abs(got - want)) <= 2.0 ** -24 * 40 * np.nanmax(np.abs(values))
+
+
+@pytest.mark.parametrize("tokens,position,dim", [(70, 10, 64), (4, 900, 64), (20, 100, 128)])
+def test_values_that_do_not_split(rt, tokens, position, dim):
+    # Keys of minus infinity weigh nothing, infinite and NaN values reach the
+    # rows that see them and no other.
+    rng = np.random.default_rng(dim + tokens)
+    heads, kv = 4, 2
+    q, keys, values = inputs(rng, tokens, position, heads, kv, dim)
+    q[:, :, 0] = np.abs(q[:, :, 0]) + 0.1
+    keys[0, 5, 0] = -np.inf
+    values[1, position + 1, 3] = np.inf
+    values[1, position + tokens - 1, 2] = np.nan
+    got = call(rt, q, keys, values, position, 0)
+    with np.errstate(all="ignore"):
+        want = exact(q, keys, values, position, 0)
+    # a weight that underflows to 0 times an infinite value is NaN on either side of f32's range
+    assert np.array_equal(np.isfinite(got), np.isfinite(want))
+    plain = np.isfinite(want)
+    assert np.max(np.abs(got[plain] - want[plain])) <= 2.0 ** -24 * 40 * 5
+
+
+@pytest.mark.parametrize("heads,kv,dim,rotary,tokens", [(14, 2, 64, 64, 5), (4, 2, 64, 32, 3), (3, 1, 80, 80, 2),
+                                                        (2, 2, 36, 24, 4), (5, 5, 64, 0, 1), (4, 1, 20, 12, 3)])
+def test_rope_append(rt, heads, kv, dim, rotary, tokens):
+    # widths of whole quads and (rotary 12) not: the same arithmetic
+    rng = np.random.default_rng(heads + dim + rotary)
+    position, capacity, half = 7, 20, rotary // 2
+    qkv = rng.standard_normal((tokens, heads + 2 * kv, dim), dtype=np.float32)
+    cos, sin = (rng.standard_normal((capacity, max(half, 1)), dtype=np.float32) for _ in range(2))
+    dq, dc, ds = (rt.DeviceArray.of(a) for a in (qkv, cos, sin))
+    q = rt.DeviceArray((heads, tokens, dim), np.float32)
+    keys, values = (rt.DeviceArray((kv, capacity, dim), np.float32).zero() for _ in range(2))
+    rt.check(rt.library().lh_rope_kv(dq.ptr, tokens, heads, kv, dim, rotary, position, dc.ptr, ds.ptr, q.ptr, keys.ptr,
+                                     values.ptr, capacity, None))
+    turned = qkv[:, :heads + kv].copy()
+    c, s = (a[position:position + tokens, None, :half] for a in (cos, sin))
+    a, b = qkv[:, :heads + kv, :half], qkv[:, :heads + kv, half:rotary]
+    turned[..., :half], turned[..., half:rotary] = a * c - b * s, b * c + a * s
+    assert np.array_equal(q.numpy(), turned[:, :heads].transpose(1, 0, 2))
+    assert np.array_equal(keys.numpy()[:, position:position + tokens], turned[:, heads:].transpose(1, 0, 2))
+    assert np.array_equal(values.numpy()[:, position:position + tokens], qkv[:, heads + kv:].transpose(1, 0, 2))
