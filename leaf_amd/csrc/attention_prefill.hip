@@ -43,7 +43,7 @@ constexpr int kStepKeys = kSlice * kSlices;
 constexpr int kRowWaves = 4;
 constexpr int kThreads = 64 * kRowWaves * kSlices;
 // Rows per wave: two MFMA tiles up to 64 values (each K and V operand read
-// from LDS then serves both; LDS would be the limit otherwise), one beyond
+// from LDS then serves both, and fewer blocks split the same keys), one beyond
 // (the split queries and outputs of two would not fit the registers).
 constexpr int row_tiles_of(int dp) { return dp <= 64 ? 2 : 1; }
 constexpr int block_rows(int dp) { return 16 * row_tiles_of(dp) * kRowWaves; }

@@ -224,7 +224,10 @@ lh_status linear_impl(const lh_weight* weight, const float* x, const int8_t* q, 
         if (c.integer_activations) {
             // quantized copy of x (when the kernel does not quantize in registers),
             // then room for 8 split-K partial sums of the output (prefill GEMM)
-            const size_t q_bytes = q ? 0 : ((tokens * c.w.cols + 255) / 256) * 256;
+            // (a given quantized input that is not 16-byte aligned is copied there
+            // for the GEMMs)
+            const bool copy_q = q && (reinterpret_cast<uintptr_t>(q) & 15) && leafhip::gemm_grouped_supported(c.w, nullptr);
+            const size_t q_bytes = q && !copy_q ? 0 : ((tokens * c.w.cols + 255) / 256) * 256;
             const size_t s_bytes = q ? 0 : ((tokens * 4 + 255) / 256) * 256;
             size_t split = tokens > 4 ? 8 * tokens * c.w.rows : 0;
             uint8_t* base = nullptr;
@@ -239,6 +242,11 @@ lh_status linear_impl(const lh_weight* weight, const float* x, const int8_t* q, 
             } else {
                 base = static_cast<uint8_t*>(
                     scratch_bytes(q_bytes + s_bytes + split * sizeof(int32_t) + 256, as_stream(stream)));
+            }
+            if (copy_q) {
+                leafhip::hip_check(hipMemcpyAsync(base, q, tokens * c.w.cols, hipMemcpyDeviceToDevice, as_stream(stream)),
+                                   "quantized input copy");
+                c.xq = reinterpret_cast<const int8_t*>(base);
             }
             if (!q) {
                 c.xq_scratch = reinterpret_cast<int8_t*>(base);

@@ -304,8 +304,8 @@ constexpr int x_plane(int q) {
 //
 // What bounds it: 2048 tokens x 5120 BF16 rows x 960 takes 68 us (was 221 with
 // f32 MFMAs): 30 us of MFMAs at the rate the card holds on such data (2.0
-// PFLOP/s at 2.06 GHz), 8 us to write the 42 MB result, the rest LDS traffic
-// (64 bytes a cycle) and the last, partly filled round of blocks.  Splitting x
+// PFLOP/s at 2.06 GHz), 8 us to write the 42 MB result, the rest the staging of
+// a stage and the last, partly filled round of blocks.  Splitting x
 // in a pass of its own measured the same (68 us, 5 of them the pass).
 template <int BITS, int MODE, bool TAIL, int MT, int NT, int WM>
 __global__ __launch_bounds__(64 * WM, 2) void gemm_f32_tiled_kernel(WeightView w, const float* __restrict__ x, int tokens,
