@@ -1902,6 +1902,14 @@ int launch_linear(const LinearCall& call, hipStream_t stream) {
     if (c.norm.kind >= 0) return -1;
     const bool group_ok = !quantized || (w.group % E == 0) || (E % w.group == 0);
     int path = c.force_path;
+    // Two to four tokens over int4 groups of whole GEMM stages: the GEMV spends
+    // its time dequantizing every weight for each token (2048 x 11264: 34, 47
+    // and 55 us against 16; 960 x 5120: 12, 18 and 22 against 5).  Up to 4096
+    // columns the GEMM's error is no larger either (0.9-1.1e-7 against 1.2e-7
+    // of the result); for other weights and longer rows it is, and they stay.
+    const bool few_int4 = w.bits == 4 && w.group < K && w.group % 32 == 0 && c.tokens > 1 && c.tokens <= 4 && K <= 4096 &&
+                          gemm_f32_supported(w, c.x);
+    if (!path && few_int4) path = 3;
     if (!path) path = (chunked && group_ok && c.tokens <= 4) ? 1 : (c.tokens > 4 && K % 4 == 0 && (!quantized || w.group % 4 == 0)) ? 3 : 2;
     if (path == 1 && !(chunked && group_ok && c.tokens <= 4)) path = 2;
     if (path == 3 && !(K % 4 == 0 && (!quantized || w.group % 4 == 0) && aligned(w.data) && aligned(c.x))) path = 2;

@@ -67,6 +67,17 @@ def test_shapes(rt, bits, group, M, K, N):
     assert within_bound(run(rt, bits, data, scales, group, bias, x), x, wd, bias)
 
 
+# Two to four tokens: int4 groups of whole stages take the GEMM too, up to 4096 columns.
+@pytest.mark.parametrize("M", [2, 3, 4])
+@pytest.mark.parametrize("K,N,group", [(64, 5, 32), (960, 1030, 64), (4096, 96, 32), (4128, 96, 32)])
+def test_few_tokens_int4(rt, M, K, N, group):
+    rng = np.random.default_rng(M + K)
+    data, scales, group, wd = weights(rng, 4, N, K, group)
+    bias = (0.1 * rng.standard_normal(N)).astype(np.float32)
+    x = rng.standard_normal((M, K), dtype=np.float32)
+    assert within_bound(run(rt, 4, data, scales, group, bias, x), x, wd, bias)
+
+
 # Rows that end inside a 32-value stage, and scale groups that are not whole stages.
 @pytest.mark.parametrize("bits,K,group", [(32, 36, 0), (32, 772, 0), (16, 100, 0), (16, 1028, 0), (8, 100, 100),
                                           (8, 96, 4), (8, 432, 48), (4, 100, 20), (4, 144, 16), (4, 1200, 100)])
