@@ -407,6 +407,7 @@ def config_benchmark(family: str, profile_steps: int = 32) -> dict:
         "prefill_ms": round(cold_ms, 2), "prefill_warm_p50_ms": round(prefill_ms, 3),
         "prefill_TFLOPs": round(flops / prefill_ms / 1e9, 2),
         "prefill_gemm": {"ms": round(gemm_ms, 3), "TFLOPs": round(gemm_tflops, 2),
+                         # of the f32 matrix instruction's rate; the GEMM splits f32 into bf16 products and passes 1
                          "frac_f32_mfma": round(gemm_tflops / F32_PEAK_TFLOPS, 4)},
         "decode_tok_s": round(1e3 / decode_ms, 1), "decode_p50_ms": round(float(np.median(step_ms)), 4),
         "decode_mean_ms": round(decode_ms, 4), "bytes_per_token": round(bytes_per_token),

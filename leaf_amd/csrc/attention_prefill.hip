@@ -69,11 +69,12 @@ __device__ __forceinline__ void block_keys(const AttentionCall& p, int group, in
 }
 
 // exp(x) for x <= 0 to about an ulp: 2^t with t = x log2(e) rounded, corrected
-// by its rounding error (six instructions; below -200 the result is 0 anyway).
+// by its rounding error (below -200 the result is 0 anyway; NaN stays NaN, so
+// that its row is found and computed again).
 __device__ __forceinline__ float exp_negative(float x) {
     constexpr float kLog2e = 1.4426950408889634f;
     constexpr float kRest = (float)(1.4426950408889634 - (double)kLog2e), kLn2 = 0.6931471805599453f;
-    x = fmaxf(x, -200.0f);
+    x = x < -200.0f ? -200.0f : x;
     const float t = x * kLog2e;
     const float rest = fmaf(x, kRest, fmaf(x, kLog2e, -t));
     const float r = __builtin_amdgcn_exp2f(t);
@@ -156,8 +157,8 @@ __global__ __launch_bounds__(kThreads) void attention_rows_kernel(AttentionCall 
     const bool partial = parts > 1;
     if (partial) {
         const int first = begin;
-        begin = first + part_index * all_steps / parts * kStepKeys;
-        end = min(end, first + (part_index + 1) * all_steps / parts * kStepKeys);
+        begin = first + int((long long)part_index * all_steps / parts) * kStepKeys;
+        end = min(end, first + int((long long)(part_index + 1) * all_steps / parts) * kStepKeys);
     }
     int t[QT], h[QT], qpos[QT];
 #pragma unroll

@@ -88,6 +88,23 @@ def test_values_that_do_not_split(rt, tokens, position, dim):
     assert np.max(np.abs(got[plain] - want[plain])) <= 2.0 ** -24 * 40 * 5
 
 
+@pytest.mark.parametrize("special", [np.nan, np.inf])
+@pytest.mark.parametrize("tokens,position,dim", [(70, 10, 64), (4, 900, 64), (20, 100, 128)])
+def test_keys_that_spoil_a_row(rt, tokens, position, dim, special):
+    # A NaN score, or one of infinity less its own maximum, makes its row NaN,
+    # as in plain f32; rows and heads that do not see the key keep their values.
+    rng = np.random.default_rng(dim + tokens)
+    q, keys, values = inputs(rng, tokens, position, 4, 2, dim)
+    q[:, :, 1] = np.abs(q[:, :, 1]) + 0.1
+    keys[1, position + tokens // 2, 1] = special
+    got = call(rt, q, keys, values, position, 0)
+    with np.errstate(all="ignore"):
+        want = exact(q, keys, values, position, 0)
+    assert np.array_equal(np.isfinite(got), np.isfinite(want)) and not np.isfinite(want).all()
+    plain = np.isfinite(want)
+    assert np.max(np.abs(got[plain] - want[plain])) <= 2.0 ** -24 * 40 * 5
+
+
 @pytest.mark.parametrize("heads,kv,dim,rotary,tokens", [(14, 2, 64, 64, 5), (4, 2, 64, 32, 3), (3, 1, 80, 80, 2),
                                                         (2, 2, 36, 24, 4), (5, 5, 64, 0, 1), (4, 1, 20, 12, 3)])
 def test_rope_append(rt, heads, kv, dim, rotary, tokens):
