@@ -90,7 +90,9 @@ __device__ __forceinline__ float visible_score(const AttentionCall& p, const flo
 }
 
 // One row's output by one wave, two passes over its keys [begin, end).  With
-// part, the unnormalized output, sum and maximum instead.
+// part, the unnormalized output, sum and maximum instead: a maximum of NaN
+// where a score is NaN, and of minus infinity with a sum of 0 where every score
+// is (other parts may hold a finite one).
 __device__ __forceinline__ void plain_row(const AttentionCall& p, int h, int t, int begin, int end, float* part) {
     const int lane = threadIdx.x & 63;
     const int kvh = h / (p.heads / p.kv_heads), qpos = p.position + t;
@@ -100,12 +102,18 @@ __device__ __forceinline__ void plain_row(const AttentionCall& p, int h, int t, 
     const float* K = p.keys + (size_t)kvh * p.capacity * p.dim;
     const float* V = p.values + (size_t)kvh * p.capacity * p.dim;
     float m = -INFINITY;
-    for (int k = begin + lane; k < end; k += 64) m = fmaxf(m, visible_score(p, q, K + (size_t)k * p.dim));
-    m = wave_max_f32(m);
+    bool nan = false;
+    for (int k = begin + lane; k < end; k += 64) {
+        const float s = visible_score(p, q, K + (size_t)k * p.dim);
+        nan = nan || s != s;
+        m = fmaxf(m, s);
+    }
+    m = __any(nan) ? NAN : wave_max_f32(m);
+    const float base = m == -INFINITY ? 0.0f : m;
     float l = 0.0f, o[2] = {0.0f, 0.0f};      // dims lane and lane + 64
     for (int k0 = begin; k0 < end; k0 += 64) {
         const int k = k0 + lane;
-        const float e = k < end ? expf(visible_score(p, q, K + (size_t)k * p.dim) - m) : 0.0f;
+        const float e = k < end ? expf(visible_score(p, q, K + (size_t)k * p.dim) - base) : 0.0f;
         l += e;
         for (int j = 0; j < min(64, end - k0); ++j) {
             const float pj = __shfl(e, j, 64);
@@ -124,7 +132,7 @@ __device__ __forceinline__ void plain_row(const AttentionCall& p, int h, int t, 
         const int d = lane + 64 * c;
         if (d >= p.dim) continue;
         if (part) part[2 + d] = o[c];
-        else p.out[((size_t)t * p.heads + h) * p.dim + d] = l > 0.0f ? o[c] / l : l == 0.0f ? 0.0f : l;
+        else p.out[((size_t)t * p.heads + h) * p.dim + d] = o[c] / l;   // a row sees a key: 0 / 0 where none has a weight
     }
 }
 
@@ -373,7 +381,9 @@ __global__ __launch_bounds__(kThreads) void attention_rows_kernel(AttentionCall 
         const float m1 = rec[4 * kDimTiles], mt = fmaxf(m[i], m1), base = mt == -INFINITY ? 0.0f : mt;
         const float a0 = exp_negative((m[i] - base) * scale2), a1 = exp_negative((m1 - base) * scale2);
         const float sum = l[i] * a0 + rec[4 * kDimTiles + 1] * a1;
-        bool bad = !finite(sum);
+        // (minus infinity: only where every score of the row's keys is)
+        const int first = p.window ? max(begin, qpos[i] + 1 - p.window) : begin;
+        bool bad = !finite(sum) || (mt == -INFINITY && first < min(end, qpos[i] + 1));
 #pragma unroll
         for (int dt = 0; dt < kDimTiles; ++dt)
 #pragma unroll
@@ -415,7 +425,10 @@ __global__ __launch_bounds__(kThreads) void attention_rows_kernel(AttentionCall 
     }
 }
 
-// Rows whose keys took several splits: their states merged, one wave a row.
+// Rows whose keys took several splits: their states merged, one wave a row.  A
+// part's NaN (maximum, sum or value) reaches the row, and a weight of 0 times
+// an infinite value is NaN, as unsplit; a row sees at least its own key, so a
+// sum of 0 means that no key has a weight, and 0 / 0 is what such a row gives.
 __global__ __launch_bounds__(256) void attention_rows_merge_kernel(AttentionCall p, int rows_per_block, int max_parts,
                                                                    int steps_per_part) {
     const int lane = threadIdx.x & 63, group = p.heads / p.kv_heads;
@@ -444,16 +457,15 @@ __global__ __launch_bounds__(256) void attention_rows_merge_kernel(AttentionCall
         float l = 0.0f, o[2] = {0.0f, 0.0f};
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-            if (mk[s] == -INFINITY) continue;
-            const float w = expf(mk[s] - m);
+            if (s >= count) break;
+            const float w = mk[s] == -INFINITY ? 0.0f : expf(mk[s] - m);
             l = fmaf(lk[s], w, l);
 #pragma unroll
             for (int c = 0; c < 2; ++c) o[c] = fmaf(v[s][c], w, o[c]);
         }
 #pragma unroll
         for (int c = 0; c < 2; ++c)
-            if (lane + 64 * c < p.dim)
-                p.out[(size_t)item * p.dim + lane + 64 * c] = l > 0.0f ? o[c] / l : l == 0.0f ? 0.0f : l;
+            if (lane + 64 * c < p.dim) p.out[(size_t)item * p.dim + lane + 64 * c] = o[c] / l;
         return;
     }
     float m = -INFINITY;
@@ -475,14 +487,14 @@ __global__ __launch_bounds__(256) void attention_rows_merge_kernel(AttentionCall
 #pragma unroll
             for (int c = 0; c < 2; ++c) {
                 const float v = lane + 64 * c < p.dim ? part[(s0 + s) * stride + 2 + lane + 64 * c] : 0.0f;
-                if (w != 0.0f) o[c] = fmaf(v, w, o[c]);
+                o[c] = fmaf(v, w, o[c]);
             }
         }
     }
     l = wave_sum_f32(l);
 #pragma unroll
     for (int c = 0; c < 2; ++c)
-        if (lane + 64 * c < p.dim) p.out[(size_t)item * p.dim + lane + 64 * c] = l > 0.0f ? o[c] / l : l == 0.0f ? 0.0f : l;
+        if (lane + 64 * c < p.dim) p.out[(size_t)item * p.dim + lane + 64 * c] = o[c] / l;
 }
 
 // How a call's keys are shared out: parts of at most a CU's share of the steps

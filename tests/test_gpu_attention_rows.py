@@ -125,3 +125,29 @@ def test_rope_append(rt, heads, kv, dim, rotary, tokens):
     assert np.array_equal(q.numpy(), turned[:, :heads].transpose(1, 0, 2))
     assert np.array_equal(keys.numpy()[:, position:position + tokens], turned[:, heads:].transpose(1, 0, 2))
     assert np.array_equal(values.numpy()[:, position:position + tokens], qkv[:, heads + kv:].transpose(1, 0, 2))
+
+
+# Rows whose visible scores in a whole part of the keys are NaN or minus
+# infinity: split over two parts, over five and more, and not split (a short
+# cache).  Row `position` is the first key of its last part in the split calls.
+@pytest.mark.parametrize("tokens,position,heads,kv,dim", [(100, 128, 2, 2, 64), (100, 512, 2, 2, 64), (4, 900, 4, 2, 64),
+                                                          (50, 128, 2, 2, 128), (20, 0, 4, 2, 64)])
+@pytest.mark.parametrize("spoilt", ["query", "own key", "every key", "masked value"])
+def test_parts_without_a_usable_score(rt, tokens, position, heads, kv, dim, spoilt):
+    rng = np.random.default_rng(tokens + position + dim)
+    q, keys, values = inputs(rng, tokens, position, heads, kv, dim)
+    q[:, :, 0] = np.abs(q[:, :, 0]) + 0.1
+    if spoilt == "query":
+        q[1, tokens // 2, 3] = np.nan
+    elif spoilt == "own key":
+        keys[0, position, 2] = np.nan
+    elif spoilt == "every key":
+        keys[0, :position + tokens, 0] = -np.inf
+    else:
+        keys[:, position, 0], values[0, position, 3] = -np.inf, np.inf      # weight 0 of an infinite value: NaN
+    got = call(rt, q, keys, values, position, 0)
+    with np.errstate(all="ignore"):
+        want = exact(q, keys, values, position, 0)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.isnan(want).any()
+    plain = np.isfinite(want)
+    assert np.max(np.abs(got[plain] - want[plain])) <= 2.0 ** -24 * 40 * 5
