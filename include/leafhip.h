@@ -188,7 +188,12 @@ lh_status lh_synchronize(void);
  * handle), at least 1 MiB per stream once used.  lh_stream_destroy waits for
  * the stream and frees that scratch; the scratch of a stream that was ever
  * captured stays allocated until the process ends, since a graph captured
- * from it may still be launched. */
+ * from it may still be launched.  Threads may call them on one stream at a time
+ * as they like: a call holds the stream's scratch until its last launch.  A graph
+ * with integer linears or one-token attention uses the scratch of the stream it
+ * was captured from: launch it in order with that stream's own calls.
+ * Attention of several tokens takes none while a stream captures (it then does
+ * not share its keys out over blocks). */
 lh_status lh_stream_create(lh_stream* out);
 lh_status lh_stream_destroy(lh_stream stream);
 lh_status lh_stream_synchronize(lh_stream stream);

@@ -7,7 +7,9 @@
 #include <cmath>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <mutex>
+#include <optional>
 #include <string>
 #include <utility>
 #include <vector>
@@ -56,29 +58,26 @@ hipStream_t as_stream(lh_stream s) { return static_cast<hipStream_t>(s); }
 
 // Device scratch of the kernel-level entry points (quantized inputs, split-K
 // sums, attention partials), one set per (device, stream): calls on different
-// streams never share memory.  A buffer that must grow is replaced and the old
-// one is kept with the stream's set, so work already queued on it, or a graph
-// captured with it, stays valid without any synchronization.  Growth while
-// the stream is capturing is refused: run the call once before capturing it.
-// lh_stream_destroy waits for the stream and frees its sets, unless the
-// stream has been captured: a graph captured from it may be launched later on
-// another stream, so such a set is kept until the process ends.  Nothing is
-// freed by static destructors, which run after the HIP runtime and a
-// profiler may have shut down.
+// streams never share memory, and a call holds its stream's set from the first
+// address it takes until its last launch, so that another thread's call on the
+// stream cannot put a launch between two of its own.  A buffer that must grow is
+// replaced and the old one is kept with the stream's set, so work already queued
+// on it, or a graph captured with it, stays valid without any synchronization.
+// Growth while the stream is capturing is refused: run the call once before
+// capturing it.  lh_stream_destroy waits for the stream and frees its sets,
+// unless the stream has been captured: a graph captured from it may be launched
+// later on another stream, so such a set is kept until the process ends.  Nothing
+// is freed by static destructors, which run after the HIP runtime and a profiler
+// may have shut down.
 struct StreamScratch {
+    std::mutex in_use;                            // held by the call that uses the buffers
     leafhip::DeviceBuffer* work = nullptr;       // grown on demand
     leafhip::DeviceBuffer* counters = nullptr;   // zeroed once; the attention kernel resets what it uses
     std::vector<leafhip::DeviceBuffer*> retired;  // outgrown work buffers
     bool captured = false;                        // a graph may hold these buffers
 };
-std::mutex g_scratch_lock;
-auto* g_scratch = new std::map<std::pair<int, hipStream_t>, StreamScratch>();
-
-StreamScratch& scratch_of(hipStream_t stream) {
-    int dev = 0;
-    leafhip::hip_check(hipGetDevice(&dev), "hipGetDevice");
-    return (*g_scratch)[{dev, stream}];
-}
+std::mutex g_scratch_lock;                        // the map, and `captured`
+auto* g_scratch = new std::map<std::pair<int, hipStream_t>, std::shared_ptr<StreamScratch>>();
 
 // Called with the stream idle and about to be destroyed.
 void release_stream_scratch(hipStream_t stream) {
@@ -88,7 +87,7 @@ void release_stream_scratch(hipStream_t stream) {
             ++it;
             continue;
         }
-        StreamScratch& sc = it->second;
+        StreamScratch& sc = *it->second;
         if (!sc.captured) {
             delete sc.work;
             delete sc.counters;
@@ -101,7 +100,7 @@ void release_stream_scratch(hipStream_t stream) {
 void mark_stream_captured(hipStream_t stream) {
     std::lock_guard<std::mutex> guard(g_scratch_lock);
     for (auto& [key, sc] : *g_scratch)
-        if (key.second == stream) sc.captured = true;
+        if (key.second == stream) sc->captured = true;
 }
 
 bool capturing(hipStream_t stream) {
@@ -110,46 +109,61 @@ bool capturing(hipStream_t stream) {
     return status != hipStreamCaptureStatusNone;
 }
 
-void* scratch_bytes(size_t bytes, hipStream_t stream) {
-    std::lock_guard<std::mutex> guard(g_scratch_lock);
-    StreamScratch& sc = scratch_of(stream);
-    if (!sc.work || sc.work->bytes < bytes) {
-        if (capturing(stream))
-            throw leafhip::Error(LH_ERROR_STATE, "Leaf decoder: kernel scratch must grow outside stream capture "
-                                                 "(run the call once before capturing it)");
-        auto* grown = new leafhip::DeviceBuffer(std::max(bytes, sc.work ? 2 * sc.work->bytes : size_t(1) << 20));
-        if (sc.work) sc.retired.push_back(sc.work);
-        sc.work = grown;
+// A stream's scratch, held by one call from here to its last launch.
+class ScratchUse {
+public:
+    explicit ScratchUse(hipStream_t stream) : stream_(stream) {
+        int dev = 0;
+        leafhip::hip_check(hipGetDevice(&dev), "hipGetDevice");
+        {
+            std::lock_guard<std::mutex> guard(g_scratch_lock);
+            auto& sc = (*g_scratch)[{dev, stream}];
+            if (!sc) sc = std::make_shared<StreamScratch>();
+            set_ = sc;
+        }
+        held_ = std::unique_lock<std::mutex>(set_->in_use);
     }
-    return sc.work->ptr;
-}
 
-// scratch_bytes for work that can also run without: null where the stream is
-// capturing and its scratch is too small.
-void* scratch_bytes_if_available(size_t bytes, hipStream_t stream) {
-    {
-        std::lock_guard<std::mutex> guard(g_scratch_lock);
-        StreamScratch& sc = scratch_of(stream);
-        if ((!sc.work || sc.work->bytes < bytes) && capturing(stream)) return nullptr;
+    void* work(size_t bytes) {
+        if (!set_->work || set_->work->bytes < bytes) {
+            if (capturing(stream_))
+                throw leafhip::Error(LH_ERROR_STATE, "Leaf decoder: kernel scratch must grow outside stream capture "
+                                                     "(run the call once before capturing it)");
+            auto* grown = new leafhip::DeviceBuffer(std::max(bytes, set_->work ? 2 * set_->work->bytes : size_t(1) << 20));
+            if (set_->work) set_->retired.push_back(set_->work);
+            set_->work = grown;
+        }
+        return set_->work->ptr;
     }
-    return scratch_bytes(bytes, stream);
-}
 
-// Zero-initialized span counters of the decode attention kernel (it resets
-// them itself), one set per (device, stream).
-unsigned* attention_counters(hipStream_t stream) {
-    std::lock_guard<std::mutex> guard(g_scratch_lock);
-    StreamScratch& sc = scratch_of(stream);
-    if (!sc.counters) {
-        if (capturing(stream))
-            throw leafhip::Error(LH_ERROR_STATE, "Leaf decoder: attention counters must be set up outside stream "
-                                                 "capture (run the call once before capturing it)");
-        auto* b = new leafhip::DeviceBuffer(1024 * sizeof(unsigned));
-        leafhip::hip_check(hipMemsetAsync(b->ptr, 0, b->bytes, stream), "hipMemsetAsync");
-        sc.counters = b;
+    // For work that can also run without: null while the stream captures (a
+    // graph that held the buffer would race, launched on another stream, with
+    // this one's calls), and on the per-thread default stream, whose one handle
+    // stands for a stream of each thread.
+    void* work_if_own(size_t bytes) {
+        if (stream_ == hipStreamPerThread || capturing(stream_)) return nullptr;
+        return work(bytes);
     }
-    return sc.counters->as<unsigned>();
-}
+
+    // Zero-initialized span counters of the decode attention kernel (it resets
+    // them itself).
+    unsigned* counters() {
+        if (!set_->counters) {
+            if (capturing(stream_))
+                throw leafhip::Error(LH_ERROR_STATE, "Leaf decoder: attention counters must be set up outside stream "
+                                                     "capture (run the call once before capturing it)");
+            auto* b = new leafhip::DeviceBuffer(1024 * sizeof(unsigned));
+            leafhip::hip_check(hipMemsetAsync(b->ptr, 0, b->bytes, stream_), "hipMemsetAsync");
+            set_->counters = b;
+        }
+        return set_->counters->as<unsigned>();
+    }
+
+private:
+    hipStream_t stream_;
+    std::shared_ptr<StreamScratch> set_;   // released after held_
+    std::unique_lock<std::mutex> held_;
+};
 
 // Numerics of this thread's kernel-level calls (lh_set_kernel_numerics).
 thread_local bool t_reference_order = false;
@@ -221,6 +235,7 @@ lh_status linear_impl(const lh_weight* weight, const float* x, const int8_t* q, 
         c.acc_out = acc;
         c.force_path = force_path;
         c.unfused_group_sum = t_reference_vnni && c.integer_activations && c.w.bits == 8 && c.w.group <= 65536;
+        std::optional<ScratchUse> scratch;
         if (c.integer_activations) {
             // quantized copy of x (when the kernel does not quantize in registers),
             // then room for 8 split-K partial sums of the output (prefill GEMM)
@@ -240,8 +255,8 @@ lh_status linear_impl(const lh_weight* weight, const float* x, const int8_t* q, 
                 base = static_cast<uint8_t*>(noalloc_scratch());
                 split = std::min(split, (LH_NOALLOC_SCRATCH_BYTES - q_bytes - s_bytes) / sizeof(int32_t));
             } else {
-                base = static_cast<uint8_t*>(
-                    scratch_bytes(q_bytes + s_bytes + split * sizeof(int32_t) + 256, as_stream(stream)));
+                scratch.emplace(as_stream(stream));
+                base = static_cast<uint8_t*>(scratch->work(q_bytes + s_bytes + split * sizeof(int32_t) + 256));
             }
             if (copy_q) {
                 leafhip::hip_check(hipMemcpyAsync(base, q, tokens * c.w.cols, hipMemcpyDeviceToDevice, as_stream(stream)),
@@ -740,15 +755,19 @@ lh_status lh_attention(const float* q_heads, const float* keys, const float* val
             leafhip::hip_check(hipGetLastError(), "attention launch");
             return;
         }
+        std::optional<ScratchUse> scratch;
         if (tokens == 1 && kv_heads <= 1024) {
             const size_t floats = ((position + tokens + 15) / 16) * heads * (dim + 2);
-            a.partial = static_cast<float*>(scratch_bytes(floats * sizeof(float), as_stream(stream)));
+            scratch.emplace(as_stream(stream));
+            a.partial = static_cast<float*>(scratch->work(floats * sizeof(float)));
             a.partial_capacity = int(floats);
-            a.counters = attention_counters(as_stream(stream));
+            a.counters = scratch->counters();
         } else if (tokens > 1 && leafhip::attention_rows_supported(a.dim)) {
             const size_t floats = leafhip::attention_rows_scratch_floats(a);
-            if (floats && floats <= 0x7fffffff)
-                a.partial = static_cast<float*>(scratch_bytes_if_available(floats * sizeof(float), as_stream(stream)));
+            if (floats && floats <= 0x7fffffff) {
+                scratch.emplace(as_stream(stream));
+                a.partial = static_cast<float*>(scratch->work_if_own(floats * sizeof(float)));
+            }
             a.partial_capacity = a.partial ? int(floats) : 0;
         }
         leafhip::check(leafhip::launch_attention(a, as_stream(stream)), "attention launch rejected", LH_ERROR_UNSUPPORTED);

@@ -1,0 +1,70 @@
+"""Scratch that several launches of one call share: who may come between them, and what runs without it.
+
+On the host, with a HIP runtime that records launches (fake_hip.py).
+"""
+from __future__ import annotations
+
+import pytest
+
+from tests.fake_hip import fake_hip  # noqa: F401  (fixture)
+
+# Calls of two and more launches over the scratch of their stream.
+CALLS = {
+    "attention of several tokens": "lambda: attention(64, 1000)",
+    "attention of one token": "lambda: attention(1, 4000)",
+    "integer linear": "lambda: lib.lh_linear(C.byref(weight(8, 256, 2048, 128)), buffer.ptr, 64, 8, buffer.ptr, None, None)",
+}
+
+
+@pytest.mark.parametrize("first", CALLS)
+@pytest.mark.parametrize("second", ["attention of several tokens", "integer linear"])
+def test_two_threads_on_one_stream(fake_hip, first, second):  # noqa: F811
+    # every call's launches follow each other: another thread's call would
+    # overwrite what the first of them left for the last
+    runs = fake_hip(f"""
+        fake.fake_set_launch_delay_us(300)
+        calls = [{CALLS[first]}, {CALLS[second]}]
+        lengths = []
+        for call in calls:
+            assert call() == 0
+            lengths.append(len(kernels()))
+        gate = threading.Barrier(2)
+        def work(call):
+            gate.wait()
+            for _ in range(20): assert call() == 0
+        threads = [threading.Thread(target=work, args=(call,)) for call in calls]
+        for t in threads: t.start()
+        for t in threads: t.join()
+        runs = []                                    # [thread, launches in a row]
+        for entry in log():
+            if entry[0] != "launch": continue
+            if runs and runs[-1][0] == entry[1]: runs[-1][1] += 1
+            else: runs.append([entry[1], 1])
+        per = {{}}
+        for thread, n in runs: per.setdefault(thread, []).append(n)
+        # a thread's calls all have one length: its runs are multiples of it
+        result = [sorted(lengths), sorted([sum(v) // 20, all(n % (sum(v) // 20) == 0 for n in v)] for v in per.values())]
+    """)
+    lengths, threads = runs
+    assert lengths[0] >= 2 and [n for n, _ in threads] == lengths
+    assert all(whole for _, whole in threads)
+
+
+def test_captured_attention_keeps_no_scratch(fake_hip):  # noqa: F811
+    # A graph may be launched on another stream, beside this stream's own
+    # calls: several tokens run unsplit in it, also where scratch is there.
+    eager, captured, per_thread = fake_hip("""
+        stream = rt.Stream()
+        assert attention(64, 1000, stream=stream.handle) == 0
+        eager = kernels()
+        fake.fake_set_capturing(1)
+        assert attention(64, 1000, stream=stream.handle) == 0
+        captured = kernels()
+        fake.fake_set_capturing(0)
+        # one handle for every thread's own default stream
+        assert attention(64, 1000, stream=2) == 0
+        result = eager, captured, kernels()
+    """)
+    assert len(eager) == 2 and "merge" in eager[1]
+    assert len(captured) == 1 and "attention_rows_kernel" in captured[0]
+    assert len(per_thread) == 1 and "attention_rows_kernel" in per_thread[0]
