@@ -138,11 +138,17 @@ public:
 
     // For work that can also run without: null while the stream captures (a
     // graph that held the buffer would race, launched on another stream, with
-    // this one's calls), and on the per-thread default stream, whose one handle
-    // stands for a stream of each thread.
+    // this one's calls), on the per-thread default stream, whose one handle
+    // stands for a stream of each thread, and where the device has no memory left.
     void* work_if_own(size_t bytes) {
         if (stream_ == hipStreamPerThread || capturing(stream_)) return nullptr;
-        return work(bytes);
+        try {
+            return work(bytes);
+        } catch (const leafhip::Error& e) {
+            if (e.code != LH_ERROR_OUT_OF_MEMORY) throw;
+            (void)hipGetLastError();   // dealt with: not the next launch's error
+            return nullptr;
+        }
     }
 
     // Zero-initialized span counters of the decode attention kernel (it resets

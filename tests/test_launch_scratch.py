@@ -68,3 +68,19 @@ def test_captured_attention_keeps_no_scratch(fake_hip):  # noqa: F811
     assert len(eager) == 2 and "merge" in eager[1]
     assert len(captured) == 1 and "attention_rows_kernel" in captured[0]
     assert len(per_thread) == 1 and "attention_rows_kernel" in per_thread[0]
+
+
+def test_attention_without_memory_for_scratch(fake_hip):  # noqa: F811
+    # splitting the keys is a choice: a call that finds no memory for it runs
+    # unsplit, and splits again once there is some
+    statuses, short, later = fake_hip("""
+        fake.fake_set_malloc_limit(1 << 16)
+        statuses = [attention(64, 1000), attention(64, 1000)]
+        short = kernels()
+        fake.fake_set_malloc_limit(1 << 40)
+        statuses.append(attention(64, 1000))
+        result = statuses, short, kernels()
+    """)
+    assert statuses == [0, 0, 0]
+    assert len(short) == 2 and all("attention_rows_kernel" in k for k in short)
+    assert len(later) == 2 and "merge" in later[1]
