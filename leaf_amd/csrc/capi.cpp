@@ -245,10 +245,7 @@ lh_status linear_impl(const lh_weight* weight, const float* x, const int8_t* q, 
         if (c.integer_activations) {
             // quantized copy of x (when the kernel does not quantize in registers),
             // then room for 8 split-K partial sums of the output (prefill GEMM)
-            // (a given quantized input that is not 16-byte aligned is copied there
-            // for the GEMMs)
-            const bool copy_q = q && (reinterpret_cast<uintptr_t>(q) & 15) && leafhip::gemm_grouped_supported(c.w, nullptr);
-            const size_t q_bytes = q && !copy_q ? 0 : ((tokens * c.w.cols + 255) / 256) * 256;
+            size_t q_bytes = q ? 0 : ((tokens * c.w.cols + 255) / 256) * 256;
             const size_t s_bytes = q ? 0 : ((tokens * 4 + 255) / 256) * 256;
             size_t split = tokens > 4 ? 8 * tokens * c.w.rows : 0;
             uint8_t* base = nullptr;
@@ -262,12 +259,20 @@ lh_status linear_impl(const lh_weight* weight, const float* x, const int8_t* q, 
                 split = std::min(split, (LH_NOALLOC_SCRATCH_BYTES - q_bytes - s_bytes) / sizeof(int32_t));
             } else {
                 scratch.emplace(as_stream(stream));
-                base = static_cast<uint8_t*>(scratch->work(q_bytes + s_bytes + split * sizeof(int32_t) + 256));
-            }
-            if (copy_q) {
-                leafhip::hip_check(hipMemcpyAsync(base, q, tokens * c.w.cols, hipMemcpyDeviceToDevice, as_stream(stream)),
-                                   "quantized input copy");
-                c.xq = reinterpret_cast<const int8_t*>(base);
+                const size_t bytes = q_bytes + s_bytes + split * sizeof(int32_t) + 256;
+                if (q && (reinterpret_cast<uintptr_t>(q) & 15) && leafhip::gemm_grouped_supported(c.w)) {
+                    // not 16-byte aligned: a copy that is reaches the faster GEMMs
+                    // (and without one the call runs all the same)
+                    const size_t copy = ((tokens * c.w.cols + 255) / 256) * 256;
+                    base = static_cast<uint8_t*>(scratch->work_if_own(copy + bytes));
+                    if (base) {
+                        leafhip::hip_check(hipMemcpyAsync(base, q, tokens * c.w.cols, hipMemcpyDeviceToDevice,
+                                                          as_stream(stream)), "quantized input copy");
+                        c.xq = reinterpret_cast<const int8_t*>(base);
+                        q_bytes = copy;
+                    }
+                }
+                if (!base) base = static_cast<uint8_t*>(scratch->work(bytes));
             }
             if (!q) {
                 c.xq_scratch = reinterpret_cast<int8_t*>(base);

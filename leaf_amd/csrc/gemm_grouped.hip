@@ -50,7 +50,10 @@ __device__ __forceinline__ void wait_vmcnt() {
 // groups end anywhere, terms fused or not, accumulators stored on request.
 // The first three have no branch inside a stage, so its four steps overlap
 // (with those branches 20 instead of 17 us for 201 tokens x 4864 x 896).
-template <int BITS, int FLUSH, int T>
+// ALIGNED false: the tokens' rows start anywhere, and come through registers,
+// which a load into LDS may not do; every stage then waits for its loads
+// (512 x 11264 x 2048, groups of 64: 104 us, 59 copied to aligned memory first).
+template <int BITS, int FLUSH, int T, bool ALIGNED = true>
 __global__ __launch_bounds__(256) void gemm_grouped_kernel(WeightView w, const int8_t* __restrict__ xq,
                                                            const float* __restrict__ xs, int tokens,
                                                            float* __restrict__ y, int epilogue,
@@ -108,9 +111,16 @@ __global__ __launch_bounds__(256) void gemm_grouped_kernel(WeightView w, const i
     auto load = [&](int stage, int buffer) {
         int8_t* base = lds + buffer * kStageBytes;
 #pragma unroll
-        for (int j = 0; j < kLoads; ++j)
-            __builtin_amdgcn_global_load_lds((void*)(src[j] + min(at0[j] + stage * step[j], last[j])),
-                                             (lds_ptr_t)(base + chunk[j] + lane * 16), 16, 0, 0);
+        for (int j = 0; j < kLoads; ++j) {
+            const int8_t* from = src[j] + min(at0[j] + stage * step[j], last[j]);
+            if (!ALIGNED && chunk[j] < kChunksX * 1024) {
+                v4i v;
+                __builtin_memcpy(&v, from, 16);
+                *(v4i*)(base + chunk[j] + lane * 16) = v;
+            } else {
+                __builtin_amdgcn_global_load_lds((void*)from, (lds_ptr_t)(base + chunk[j] + lane * 16), 16, 0, 0);
+            }
+        }
         __builtin_amdgcn_global_load_lds((void*)(scale_row + group_of(stage, scale_end)),
                                          (lds_ptr_t)(base + kChunks * 1024 + wave * 256 + lane * 4), 4, 0, 0);
     };
@@ -166,7 +176,7 @@ __global__ __launch_bounds__(256) void gemm_grouped_kernel(WeightView w, const i
     int left = group_steps;                                   // steps until the group ends (FLUSH 0 and 4)
     auto run_stage = [&](int s, auto tail) {                  // tail: fewer than four steps
         constexpr bool kTail = decltype(tail)::value;
-        wait_vmcnt<(kStages - 2) * (kLoads + 1)>();
+        wait_vmcnt<ALIGNED ? (kStages - 2) * (kLoads + 1) : 0>();
         lds_barrier();                                        // stage s landed; stage s - 1 is no longer read
         load(s + kStages - 1, (s + kStages - 1) % kStages);
         const int8_t* base = lds + (s % kStages) * kStageBytes;
@@ -244,18 +254,20 @@ __global__ __launch_bounds__(256) void gemm_grouped_kernel(WeightView w, const i
     }
 }
 
-template <int BITS, int FLUSH, int T>
+template <int BITS, int FLUSH, int T, bool ALIGNED = true>
 void launch_tiles(const WeightView& w, const int8_t* xq, const float* xs, int tokens, float* y, int epilogue,
                   int32_t* acc_out, int unfused, hipStream_t stream) {
     const int m_tiles = (tokens + 32 * T - 1) / (32 * T), n_tiles = (w.rows + 32 * T - 1) / (32 * T);
-    gemm_grouped_kernel<BITS, FLUSH, T><<<m_tiles * n_tiles, 256, 0, stream>>>(w, xq, xs, tokens, y, epilogue, acc_out,
+    gemm_grouped_kernel<BITS, FLUSH, T, ALIGNED><<<m_tiles * n_tiles, 256, 0, stream>>>(w, xq, xs, tokens, y, epilogue, acc_out,
                                                                               unfused, m_tiles);
 }
 
 template <int BITS, int T>
 void launch_flush(const WeightView& w, const int8_t* xq, const float* xs, int tokens, float* y, int epilogue,
                   int32_t* acc_out, int unfused, hipStream_t stream) {
-    if (unfused || acc_out) launch_tiles<BITS, 0, T>(w, xq, xs, tokens, y, epilogue, acc_out, unfused, stream);
+    if (reinterpret_cast<uintptr_t>(xq) & 15)
+        launch_tiles<BITS, 0, T, false>(w, xq, xs, tokens, y, epilogue, acc_out, unfused, stream);
+    else if (unfused || acc_out) launch_tiles<BITS, 0, T>(w, xq, xs, tokens, y, epilogue, acc_out, unfused, stream);
     else if (w.group == 32) launch_tiles<BITS, 1, T>(w, xq, xs, tokens, y, epilogue, acc_out, unfused, stream);
     else if (w.group == 64) launch_tiles<BITS, 2, T>(w, xq, xs, tokens, y, epilogue, acc_out, unfused, stream);
     else if (w.group % kStageK == 0) launch_tiles<BITS, 4, T>(w, xq, xs, tokens, y, epilogue, acc_out, unfused, stream);
@@ -264,10 +276,9 @@ void launch_flush(const WeightView& w, const int8_t* xq, const float* xs, int to
 
 }  // namespace
 
-bool gemm_grouped_supported(const WeightView& w, const int8_t* xq) {
-    auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+bool gemm_grouped_supported(const WeightView& w) {
     return (w.bits == 8 || w.bits == 4) && w.cols > 0 && w.group > 0 && w.group % 32 == 0 && w.cols % w.group == 0 &&
-           aligned(w.data) && aligned(xq);
+           (reinterpret_cast<uintptr_t>(w.data) & 15) == 0;
 }
 
 void launch_gemm_grouped(const WeightView& w, const int8_t* xq, const float* xs, int tokens, float* y, int epilogue,

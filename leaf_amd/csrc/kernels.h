@@ -121,8 +121,9 @@ void launch_gemm_w8a8_mfma(const int8_t* W, const float* w_scales, const float* 
                            const GemmTiles& tiles, int32_t* partial, hipStream_t stream);
 
 // Integer-activation GEMM for int8 / int4 weights with scale groups of whole
-// multiples of 32 values (gemm_grouped.hip), 16-byte aligned operands.
-bool gemm_grouped_supported(const WeightView& w, const int8_t* xq);
+// multiples of 32 values (gemm_grouped.hip), weights 16-byte aligned; an input
+// that is not takes a slower kernel of the same results.
+bool gemm_grouped_supported(const WeightView& w);
 void launch_gemm_grouped(const WeightView& w, const int8_t* xq, const float* xs, int tokens, float* y, int epilogue,
                          int32_t* acc_out, bool unfused, hipStream_t stream);
 

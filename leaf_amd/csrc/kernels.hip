@@ -1833,9 +1833,10 @@ int launch_linear(const LinearCall& call, hipStream_t stream) {
         const bool per_row = w.group == K;
         const bool fast = per_row && chunked;
         int path = c.force_path;
-        // the input as the GEMMs will see it: given, or quantized into the scratch
-        const bool gemm = (per_row && w.bits == 8 && gemm_w8a8_mfma_supported(K) && aligned(w.data)) ||
-                          gemm_grouped_supported(w, c.xq ? c.xq : c.xq_scratch);
+        // (the per-row GEMM loads the input 16 bytes at a time straight into LDS)
+        const bool gemm_per_row = per_row && w.bits == 8 && gemm_w8a8_mfma_supported(K) && aligned(w.data) &&
+                                  aligned(c.xq ? c.xq : c.xq_scratch);
+        const bool gemm = gemm_per_row || gemm_grouped_supported(w);
         if (!path) path = (fast && c.tokens <= 4) ? 1 : gemm && (c.tokens > 4 || !per_row) ? 3 : 2;
         if (path == 1 && !(fast && c.tokens <= 4)) path = 2;
         if (path == 3 && !gemm) path = 2;
@@ -1858,7 +1859,7 @@ int launch_linear(const LinearCall& call, hipStream_t stream) {
             if (w.bits == 8) launch_gemv_int<8>(c, xq, xs, stream); else launch_gemv_int<4>(c, xq, xs, stream);
             return 1;
         }
-        if (path == 3 && per_row && w.bits == 8 && gemm_w8a8_mfma_supported(K)) {
+        if (path == 3 && gemm_per_row) {
             const GemmTiles tiles = gemm_w8a8_tiles(c.tokens, w.rows, K, c.split_scratch ? c.split_capacity : 0);
             int32_t* partial = tiles.splits > 1 ? c.split_scratch : nullptr;
             const int splits = tiles.splits;

@@ -39,7 +39,7 @@ def kernels():
     """The kernels launched since the last call: their mangled names."""
     return [e[2] for e in log() if e[0] == "launch"]
 
-buffer = rt.DeviceArray((1 << 16,), np.float32)     # an address: no kernel runs
+buffer = rt.DeviceArray((1 << 20,), np.float32)     # an address: no kernel runs
 
 def attention(tokens, position, heads=14, kv=2, dim=64, window=0, stream=None, q=None, out=None):
     return lib.lh_attention(q or buffer.ptr, buffer.ptr, buffer.ptr, position + tokens, heads, kv, dim, tokens,

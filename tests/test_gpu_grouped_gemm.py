@@ -61,3 +61,39 @@ def test_grouped_gemm_bit_exact(rt, oracle, bits, K, group, M, N):
     dy.zero()
     rt.check(rt.library().lh_linear_q(C.byref(dw.desc), dq.ptr + 4, ds.ptr, M, dy.ptr, None, None))
     assert np.array_equal(dy.numpy().view(np.uint32), expected.view(np.uint32))
+
+
+# An input that is not aligned and may not be copied (the stream captures): every
+# weight width and kind of group, rows that end inside a stage, both block sizes.
+@pytest.mark.parametrize("bits,K,group", [(8, 96, 32), (8, 2048, 128), (8, 960, 960), (4, 896, 32), (4, 288, 96)])
+@pytest.mark.parametrize("M,N,offset", [(5, 97, 1), (33, 256, 4), (300, 3100, 7), (513, 1030, 8)])
+def test_captured_unaligned_input_bit_exact(rt, oracle, bits, K, group, M, N, offset):
+    rng = np.random.default_rng(bits * 1000 + K + M)
+    wq, ws = quantize((0.02 * rng.standard_normal((N, K))).astype(np.float32), bits, group)
+    bias = rng.standard_normal(N, dtype=np.float32)
+    x = rng.standard_normal((M, K), dtype=np.float32)
+    dw = rt.DeviceWeight(wq, bits, K, ws, group, bias)
+    q, _ = oracle.quantize_rows(x)
+    oracle.set_vnni_policy(0)
+    expected = oracle.linear_int(bits, N, K, group, wq, ws, bias, x)
+    dq = rt.DeviceArray.of(np.concatenate([np.zeros(offset, np.int8), q.reshape(-1)]))
+    ds = rt.DeviceArray.of(np.maximum(np.abs(x).max(axis=1) / np.float32(127), np.float32(1e-12)).astype(np.float32))
+    dy, dacc = rt.DeviceArray((M, N), np.float32), rt.DeviceArray((M, N, K // group), np.int32)
+    stream = rt.Stream()
+
+    def call():
+        rt.check(rt.library().lh_linear_q(C.byref(dw.desc), dq.ptr + offset, ds.ptr, M, dy.ptr, dacc.ptr, stream.handle))
+
+    call()                                             # sizes the stream's scratch
+    stream.synchronize()
+    graph = rt.Graph(stream, call)
+    for _ in range(2):
+        dy.zero()
+        dacc.zero()
+        rt.synchronize()
+        graph.launch()
+        stream.synchronize()
+        assert np.array_equal(dy.numpy().view(np.uint32), expected.view(np.uint32))
+        assert np.array_equal(dacc.numpy(), oracle.int_accumulators(bits, N, K, group, wq, q))
+    graph.close()
+    stream.close()

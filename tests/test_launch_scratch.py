@@ -84,3 +84,32 @@ def test_attention_without_memory_for_scratch(fake_hip):  # noqa: F811
     assert statuses == [0, 0, 0]
     assert len(short) == 2 and all("attention_rows_kernel" in k for k in short)
     assert len(later) == 2 and "merge" in later[1]
+
+
+def test_unaligned_quantized_input(fake_hip):  # noqa: F811
+    # copied to where the faster GEMMs can load it, except into a graph or
+    # where there is no memory: a kernel takes it as it is
+    result = fake_hip("""
+        stream = rt.Stream()
+        def call(group): return lib.lh_linear_q(C.byref(weight(8, 256, 2048, group)), buffer.ptr + 4, buffer.ptr, 64,
+                                                buffer.ptr, None, stream.handle)
+        def what(): return [e[0] if e[0] == "copy" else e[2] for e in log()]
+        result = []
+        for group in (128, 2048):
+            assert call(group) == 0
+            eager = what()
+            fake.fake_set_capturing(1)
+            assert call(group) == 0
+            captured = what()
+            fake.fake_set_capturing(0)
+            result.append([eager, captured])
+        fake.fake_set_malloc_limit(1 << 21)
+        big = lambda: lib.lh_linear_q(C.byref(weight(8, 64, 2048, 128)), buffer.ptr + 4, buffer.ptr, 1000, buffer.ptr,
+                                      None, stream.handle)
+        result.append([big(), what()])
+    """)
+    for eager, captured in result[:2]:
+        assert eager[0] == "copy" and "gemm" in eager[1]
+        assert len(captured) == 1 and "gemm_grouped_kernel" in captured[0] and "Lb0E" in captured[0]
+    status, launched = result[2]
+    assert status == 0 and len(launched) == 1 and "Lb0E" in launched[0]
