@@ -557,7 +557,11 @@ void launch_rows(const AttentionCall& call, hipStream_t stream) {
 
 }  // namespace
 
-bool attention_rows_supported(int dim) { return dim > 0 && dim <= 128 && dim % 4 == 0; }
+bool attention_rows_supported(const AttentionCall& call) {
+    auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    return call.tokens > 1 && call.dim > 0 && call.dim <= 128 && call.dim % 4 == 0 && aligned(call.q_heads) &&
+           aligned(call.keys) && aligned(call.values) && aligned(call.out);
+}
 
 size_t attention_rows_scratch_floats(const AttentionCall& call) {
     RowsPlan plan;

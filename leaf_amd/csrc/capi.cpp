@@ -773,7 +773,7 @@ lh_status lh_attention(const float* q_heads, const float* keys, const float* val
             a.partial = static_cast<float*>(scratch->work(floats * sizeof(float)));
             a.partial_capacity = int(floats);
             a.counters = scratch->counters();
-        } else if (tokens > 1 && leafhip::attention_rows_supported(a.dim)) {
+        } else if (leafhip::attention_rows_supported(a)) {
             const size_t floats = leafhip::attention_rows_scratch_floats(a);
             if (floats && floats <= 0x7fffffff) {
                 scratch.emplace(as_stream(stream));

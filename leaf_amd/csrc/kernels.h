@@ -178,8 +178,8 @@ struct AttentionCall {
 bool launch_attention(const AttentionCall& call, hipStream_t stream);
 
 // Attention of several tokens on the bf16 matrix cores (attention_prefill.hip),
-// head dims up to 128 in multiples of 4.
-bool attention_rows_supported(int dim);
+// head dims up to 128 in multiples of 4, queries, keys, values and outputs 16-byte aligned.
+bool attention_rows_supported(const AttentionCall& call);
 // Floats of `partial` with which a call splits its keys over blocks as it would
 // like to (0: not at all); with fewer it runs unsplit.
 size_t attention_rows_scratch_floats(const AttentionCall& call);

@@ -1981,7 +1981,7 @@ bool launch_attention(const AttentionCall& call, hipStream_t stream) {
         }
         if (splits == 1) per_split = total;
     }
-    if (call.tokens > 1 && attention_rows_supported(call.dim)) {
+    if (attention_rows_supported(call)) {
         launch_attention_rows(call, stream);
         return true;
     }

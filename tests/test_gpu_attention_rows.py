@@ -151,3 +151,18 @@ def test_parts_without_a_usable_score(rt, tokens, position, heads, kv, dim, spoi
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.isnan(want).any()
     plain = np.isfinite(want)
     assert np.max(np.abs(got[plain] - want[plain])) <= 2.0 ** -24 * 40 * 5
+
+
+@pytest.mark.parametrize("tokens,position,heads,kv,dim,window", [(33, 191, 4, 1, 64, 0), (20, 1000, 6, 3, 128, 0),
+                                                                 (64, 0, 6, 2, 80, 33)])
+def test_unaligned_arrays(rt, tokens, position, heads, kv, dim, window):
+    # every array one float past a 16-byte boundary
+    rng = np.random.default_rng(tokens + dim)
+    arrays = inputs(rng, tokens, position, heads, kv, dim)
+    q, keys, values = arrays
+    dq, dk, dv = (rt.DeviceArray.of(np.concatenate([np.zeros(1, np.float32), a.reshape(-1)])) for a in arrays)
+    out = rt.DeviceArray((1 + tokens * heads * dim,), np.float32).zero()
+    rt.check(rt.library().lh_attention(dq.ptr + 4, dk.ptr + 4, dv.ptr + 4, keys.shape[1], heads, kv, dim, tokens, position,
+                                       window, out.ptr + 4, None))
+    got, want = out.numpy()[1:].reshape(tokens, heads, dim), exact(q, keys, values, position, window)
+    assert np.max(np.abs(got - want)) <= 2.0 ** -24 * 40 * np.nanmax(np.abs(values))
