@@ -1137,11 +1137,12 @@ __global__ __launch_bounds__(kBlock) void attention_kernel(AttentionCall p, int 
         const float block_max = block_reduce<float>(local_max, red, [](float a, float b) { return fmaxf(a, b); },
                                                     wave_max_f32);
         const float m_new = fmaxf(m, block_max);
+        const float base = m_new == -INFINITY ? 0.0f : m_new;   // no finite score yet: every weight is 0 (NaN stays NaN)
         const float alpha = m == -INFINITY ? 0.0f : expf(m - m_new);
         __syncthreads();
         float e = 0.0f;
         if (threadIdx.x < n) {
-            e = expf(scores[threadIdx.x] - m_new);
+            e = expf(scores[threadIdx.x] - base);
             scores[threadIdx.x] = e;
         }
         const float block_sum = block_reduce<float>(e, red, [](float a, float b) { return a + b; }, wave_sum_f32);
@@ -1172,7 +1173,7 @@ __global__ __launch_bounds__(kBlock) void attention_kernel(AttentionCall p, int 
         float* out = p.out + ((size_t)t * p.heads + h) * dim;
         for (int d = threadIdx.x; d < dim; d += blockDim.x) {
             const float v = (o_s[0][d] + o_s[1][d]) + (o_s[2][d] + o_s[3][d]);
-            out[d] = l > 0.0f ? v / l : 0.0f;
+            out[d] = v / l;   // NaN of a score or value included; 0 / 0 where no key has a weight
         }
     } else {
         float* part = p.partial + (((size_t)t * p.heads + h) * gridDim.z + split) * (dim + 2);

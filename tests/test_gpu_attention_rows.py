@@ -166,3 +166,31 @@ def test_unaligned_arrays(rt, tokens, position, heads, kv, dim, window):
                                        window, out.ptr + 4, None))
     got, want = out.numpy()[1:].reshape(tokens, heads, dim), exact(q, keys, values, position, window)
     assert np.max(np.abs(got - want)) <= 2.0 ** -24 * 40 * np.nanmax(np.abs(values))
+
+
+# The general kernel (head dims beyond 128, arrays that are not aligned): NaN
+# and minus infinity as in the kernel above, also where the first 256 keys have
+# no weight.
+@pytest.mark.parametrize("dim,offset", [(160, 0), (64, 1)])
+@pytest.mark.parametrize("spoilt", ["query", "key", "early keys", "every key"])
+def test_general_kernel_without_a_usable_score(rt, dim, offset, spoilt):
+    tokens, position, heads, kv = 20, 300, 4, 2
+    rng = np.random.default_rng(dim)
+    q, keys, values = inputs(rng, tokens, position, heads, kv, dim)
+    q[:, :, 0] = np.abs(q[:, :, 0]) + 0.1
+    if spoilt == "query":
+        q[1, 7, 3] = np.nan
+    elif spoilt == "key":
+        keys[0, position + 4, 2] = np.nan
+    else:
+        keys[0, :position + tokens if spoilt == "every key" else 290, 0] = -np.inf
+    dq, dk, dv = (rt.DeviceArray.of(np.concatenate([np.zeros(offset, np.float32), a.reshape(-1)])) for a in (q, keys, values))
+    out = rt.DeviceArray((tokens, heads, dim), np.float32)
+    rt.check(rt.library().lh_attention(dq.ptr + 4 * offset, dk.ptr + 4 * offset, dv.ptr + 4 * offset, keys.shape[1], heads,
+                                       kv, dim, tokens, position, 0, out.ptr, None))
+    got = out.numpy()
+    with np.errstate(all="ignore"):
+        want = exact(q, keys, values, position, 0)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    plain = np.isfinite(want)
+    assert np.max(np.abs(got[plain] - want[plain])) <= 2.0 ** -24 * 40 * 5
