@@ -1097,10 +1097,19 @@ __global__ __launch_bounds__(kBlock) void rope_kv_quads_kernel(RopeKvCall p) {
 // transformer.cpp:94-146).  Scores use the CPU's sequential dot order and
 // (dot * scale) * scale; the softmax is rescaled per key block, so results
 // agree with the CPU's max / exp / sum / divide to rounding.
+// kFew...: calls over a few dozen keys that could take the matrix cores' kernel.
+// As exact as there: eight fused chains added at the end (one in
+// 64 bits up to 32 dims), the scale applied to their distance from the maximum.
+// 16 tokens behind 20 keys, relative to 64 bits, the matrix cores' kernel second:
+// 1.6e-7 against 2.3e-7 for heads of 128, 1.4e-7 and 1.7e-7 (64), 1.1e-7 both
+// (32).  (Over many keys the chains cost more than they give: 300 tokens of 8
+// heads of 160 behind 500 keys 298 instead of 245 us.)
 // Grid: (heads, tokens, splits).  With splits > 1 (decode) each block writes
 // (max, sum, o[dim]) for its key range to `partial`, merged by attention_merge.
 constexpr int kKeysPerPass = 256;
 
+enum ScoreSum : int { kSequential, kFewChains, kFewDouble };
+template <int SCORE>
 __global__ __launch_bounds__(kBlock) void attention_kernel(AttentionCall p, int keys_per_split) {
     __shared__ float q_s[256];
     __shared__ float scores[kKeysPerPass];
@@ -1120,6 +1129,7 @@ __global__ __launch_bounds__(kBlock) void attention_kernel(AttentionCall p, int 
     const float* K = p.keys + (size_t)kvh * p.capacity * dim;
     const float* V = p.values + (size_t)kvh * p.capacity * dim;
     float m = -INFINITY, l = 0.0f;
+    const float scale2 = SCORE != kSequential ? p.scale * p.scale : 1.0f;       // what scores are still to be multiplied by
     // thread owns output dims d = tid % 64 (+64, ...) for key lane kl = tid / 64
     const int dl = threadIdx.x & 63, kl = threadIdx.x >> 6;
     float o[4] = {0.f, 0.f, 0.f, 0.f};   // dims dl, dl+64, dl+128, dl+192
@@ -1128,21 +1138,38 @@ __global__ __launch_bounds__(kBlock) void attention_kernel(AttentionCall p, int 
         float local_max = -INFINITY;
         if (threadIdx.x < n) {
             const float* krow = K + (size_t)(k0 + threadIdx.x) * dim;
-            float sum = 0.0f;
-            for (int d = 0; d < dim; ++d) sum = sum + q_s[d] * krow[d];
-            const float sc = sum * p.scale * p.scale;
-            scores[threadIdx.x] = sc;
-            local_max = sc;
+            float sum;
+            if constexpr (SCORE == kSequential) {
+                sum = 0.0f;
+                for (int d = 0; d < dim; ++d) sum = sum + q_s[d] * krow[d];
+                sum = sum * p.scale * p.scale;
+            } else if constexpr (SCORE == kFewDouble) {
+                double part = 0.0;
+                for (int d = 0; d < dim; ++d) part = fma((double)q_s[d], (double)krow[d], part);
+                sum = (float)part;
+            } else {
+                float part[8] = {};
+                int d = 0;
+                for (; d + 8 <= dim; d += 8)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) part[j] = fmaf(q_s[d + j], krow[d + j], part[j]);
+#pragma unroll
+                for (int j = 0; j < 7; ++j)
+                    if (d + j < dim) part[j] = fmaf(q_s[d + j], krow[d + j], part[j]);
+                sum = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
+            }
+            scores[threadIdx.x] = sum;
+            local_max = sum;
         }
         const float block_max = block_reduce<float>(local_max, red, [](float a, float b) { return fmaxf(a, b); },
                                                     wave_max_f32);
         const float m_new = fmaxf(m, block_max);
         const float base = m_new == -INFINITY ? 0.0f : m_new;   // no finite score yet: every weight is 0 (NaN stays NaN)
-        const float alpha = m == -INFINITY ? 0.0f : expf(m - m_new);
+        const float alpha = m == -INFINITY ? 0.0f : expf((m - m_new) * scale2);
         __syncthreads();
         float e = 0.0f;
         if (threadIdx.x < n) {
-            e = expf(scores[threadIdx.x] - base);
+            e = expf((scores[threadIdx.x] - base) * scale2);
             scores[threadIdx.x] = e;
         }
         const float block_sum = block_reduce<float>(e, red, [](float a, float b) { return a + b; }, wave_sum_f32);
@@ -1982,12 +2009,18 @@ bool launch_attention(const AttentionCall& call, hipStream_t stream) {
         }
         if (splits == 1) per_split = total;
     }
+    // Over a few dozen keys one block per head and token ends before the matrix
+    // cores' kernel has staged its first 64 keys (4 tokens of 32 heads of 128: 4.9
+    // against 8.7 us at once, 7.5 against 9.2 behind 32 keys).  They meet at 40 to
+    // 50 keys, for all head dims from 20 to 128 but 64, where it is later.
+    dim3 grid(call.heads, call.tokens, splits);
     if (attention_rows_supported(call)) {
-        launch_attention_rows(call, stream);
+        if (total > 40) launch_attention_rows(call, stream);
+        else if (call.dim > 32) attention_kernel<kFewChains><<<grid, kBlock, 0, stream>>>(call, per_split);
+        else attention_kernel<kFewDouble><<<grid, kBlock, 0, stream>>>(call, per_split);
         return true;
     }
-    dim3 grid(call.heads, call.tokens, splits);
-    attention_kernel<<<grid, kBlock, 0, stream>>>(call, per_split);
+    attention_kernel<kSequential><<<grid, kBlock, 0, stream>>>(call, per_split);
     if (splits > 1) attention_merge_kernel<<<dim3(call.heads, call.tokens), 64, 0, stream>>>(call, splits);
     return true;
 }

@@ -194,3 +194,18 @@ def test_general_kernel_without_a_usable_score(rt, dim, offset, spoilt):
     assert np.array_equal(np.isnan(got), np.isnan(want))
     plain = np.isfinite(want)
     assert np.max(np.abs(got[plain] - want[plain])) <= 2.0 ** -24 * 40 * 5
+
+
+# Up to 40 keys (one block per head and token) and just beyond, with windows,
+# dims with and without a remainder of eight, and a NaN in between.
+@pytest.mark.parametrize("tokens,position,heads,kv,dim,window", [
+    (2, 0, 12, 12, 64, 0), (40, 0, 4, 2, 128, 0), (17, 23, 6, 2, 80, 9), (5, 35, 8, 1, 32, 0), (3, 20, 4, 4, 36, 5),
+    (40, 0, 3, 3, 4, 0), (41, 0, 3, 3, 4, 0), (9, 32, 4, 2, 128, 12)])
+def test_few_keys(rt, tokens, position, heads, kv, dim, window):
+    rng = np.random.default_rng(tokens + dim)
+    q, keys, values = inputs(rng, tokens, position, heads, kv, dim)
+    q[0, tokens // 2, 0] = np.nan
+    got, want = call(rt, q, keys, values, position, window), exact(q, keys, values, position, window)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.isnan(want).any()
+    plain = np.isfinite(want)
+    assert np.max(np.abs(got[plain] - want[plain])) <= 2.0 ** -24 * 40 * np.nanmax(np.abs(values))

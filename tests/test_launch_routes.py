@@ -17,4 +17,14 @@ def test_attention_alignment(fake_hip, argument):  # noqa: F811
         result = aligned, kernels()
     """)
     assert "attention_rows_kernel" in aligned[0]
-    assert len(unaligned) == 1 and "16attention_kernel" in unaligned[0]
+    assert len(unaligned) == 1 and "16attention_kernelILi0E" in unaligned[0]
+
+
+@pytest.mark.parametrize("tokens,position,small", [(2, 0, True), (4, 36, True), (40, 0, True), (2, 39, False), (41, 0, False)])
+@pytest.mark.parametrize("heads,kv,dim", [(32, 8, 128), (8, 1, 32), (14, 2, 64)])
+def test_attention_over_few_keys(fake_hip, heads, kv, dim, tokens, position, small):  # noqa: F811
+    launched = fake_hip(f"""
+        assert attention({tokens}, {position}, {heads}, {kv}, {dim}) == 0
+        result = kernels()
+    """)
+    assert len(launched) == 1 and (f"16attention_kernelILi{1 if dim > 32 else 2}E" if small else "attention_rows_kernel") in launched[0]
