@@ -28,6 +28,7 @@
 // 64 over 2 KV heads take 81 us (124 with f32 MFMAs), 256 tokens of 32 heads of
 // 128 behind 1000 keys 54 us (905 in a kernel without MFMAs).
 #include <algorithm>
+#include <cstdint>
 #include <type_traits>
 
 #include "device_common.h"
@@ -500,13 +501,18 @@ __global__ __launch_bounds__(256) void attention_rows_merge_kernel(AttentionCall
 // How a call's keys are shared out: parts of at most a CU's share of the steps
 // (and at least two steps), as many to a tile as it needs, equal within it.
 // Half that size costs more in blocks and partial results than it evens out
-// (512 tokens, 32 heads of 64: 47 instead of 37 us).
+// (512 tokens, 32 heads of 64: 47 instead of 37 us).  Parts grow until their
+// results fit in max_floats.
 struct RowsPlan {
     int row_tiles = 0;
     RowItems items;
 };
 
-void plan_rows(const AttentionCall& call, RowsPlan& plan) {
+size_t partial_floats(const AttentionCall& call, int max_parts) {
+    return (size_t)max_parts * call.tokens * call.heads * (call.dim + 2);
+}
+
+void plan_rows(const AttentionCall& call, size_t max_floats, RowsPlan& plan) {
     const int group = call.heads / call.kv_heads, rows = call.tokens * group;
     const int per_block = block_rows((call.dim + 31) / 32 * 32);
     plan.row_tiles = (rows + per_block - 1) / per_block;
@@ -521,7 +527,8 @@ void plan_rows(const AttentionCall& call, RowsPlan& plan) {
         total += steps[tile];
         longest = std::max(longest, steps[tile]);
     }
-    const int per = (int)std::max<long>(2, (total * call.kv_heads + 255) / 256);
+    int per = (int)std::max<long>(2, (total * call.kv_heads + 255) / 256);
+    while (parts_of(longest, per) > 1 && partial_floats(call, parts_of(longest, per)) > max_floats) per += (per + 3) / 4;
     if (parts_of(longest, per) == 1) return;
     int count = 0;
     for (int tile = 0; tile < plan.row_tiles; ++tile) {
@@ -539,15 +546,10 @@ void plan_rows(const AttentionCall& call, RowsPlan& plan) {
     items.steps_per_part = per;
 }
 
-size_t partial_floats(const AttentionCall& call, const RowsPlan& plan) {
-    return plan.items.count ? (size_t)plan.items.max_parts * call.tokens * call.heads * (call.dim + 2) : 0;
-}
-
 template <int DP>
 void launch_rows(const AttentionCall& call, hipStream_t stream) {
     RowsPlan plan;
-    plan_rows(call, plan);
-    if (!call.partial || partial_floats(call, plan) > (size_t)call.partial_capacity) plan.items.count = 0;
+    plan_rows(call, call.partial ? (size_t)call.partial_capacity : 0, plan);
     const int items = plan.items.count ? plan.items.count : plan.row_tiles;
     attention_rows_kernel<DP><<<items * call.kv_heads, kThreads, 0, stream>>>(call, plan.row_tiles, plan.items);
     if (plan.items.count)
@@ -565,8 +567,17 @@ bool attention_rows_supported(const AttentionCall& call) {
 
 size_t attention_rows_scratch_floats(const AttentionCall& call) {
     RowsPlan plan;
-    plan_rows(call, plan);
-    return partial_floats(call, plan);
+    plan_rows(call, SIZE_MAX, plan);
+    return plan.items.count ? partial_floats(call, plan.items.max_parts) : 0;
+}
+
+// The longest tile's steps are at most 2 / (tiles + 1) of a KV head's, so it has
+// at most 512 / (kv_heads (tiles + 1)) + 1 parts, and one where kv_heads tiles
+// reach 512; each holds a row of dim + 2 floats for all tiles * rows of them.
+size_t attention_rows_scratch_limit(int tokens, int heads, int kv_heads, int dim) {
+    const size_t per_block = block_rows((dim + 31) / 32 * 32);
+    const size_t tiles = ((size_t)tokens * (heads / kv_heads) + per_block - 1) / per_block * kv_heads;
+    return (512 + std::min<size_t>(tiles, 512)) * per_block * (dim + 2);
 }
 
 void launch_attention_rows(const AttentionCall& call, hipStream_t stream) {

@@ -181,8 +181,11 @@ bool launch_attention(const AttentionCall& call, hipStream_t stream);
 // head dims up to 128 in multiples of 4, queries, keys, values and outputs 16-byte aligned.
 bool attention_rows_supported(const AttentionCall& call);
 // Floats of `partial` with which a call splits its keys over blocks as it would
-// like to (0: not at all); with fewer it runs unsplit.
+// like to (0: not at all); with fewer it splits less.
 size_t attention_rows_scratch_floats(const AttentionCall& call);
+// As many as any call of up to `tokens` tokens asks for, wherever it stands: at
+// most 35 MB.
+size_t attention_rows_scratch_limit(int tokens, int heads, int kv_heads, int dim);
 void launch_attention_rows(const AttentionCall& call, hipStream_t stream);
 
 // act = up * activate(gate) for gated MLPs, act = activate(up) otherwise.

@@ -198,6 +198,17 @@ void Session::plan(uint32_t tokens, bool all_logits) {
         // split-K sums of the W8A8 prefill GEMM: up to 8 splits of a
         // hidden-wide output (wider outputs split less or not at all)
         if (model.activation_bits == 8 && tokens > 4) grow<int32_t>(split_, P * 8 * c.hidden);
+        // partial results of a prompt's attention, its keys shared out over blocks;
+        // without memory for them it runs unsplit
+        if (tokens > 1 && !reference_ && c.head_dim <= 128) {
+            try {
+                grow<float>(rows_partial_, attention_rows_scratch_limit(int(tokens), int(c.heads), int(c.kv_heads),
+                                                                        int(c.head_dim)));
+            } catch (const Error& e) {
+                if (e.code != LH_ERROR_OUT_OF_MEMORY) throw;
+                (void)hipGetLastError();
+            }
+        }
         grow<uint32_t>(ids_, P);
         if (host_ids_) (void)hipHostFree(host_ids_);
         hip_check(hipHostMalloc((void**)&host_ids_, P * sizeof(uint32_t)), "hipHostMalloc");
@@ -793,7 +804,8 @@ void Session::launch(int M, size_t position, bool all_logits, const int* positio
         at.q_heads = q_heads_.as<float>(); at.keys = keys; at.values = values; at.out = attn_.as<float>();
         at.heads = int(c.heads); at.kv_heads = int(c.kv_heads); at.tokens = M; at.position = int(position);
         at.dim = dim; at.capacity = int(capacity); at.window = int(c.sliding_window); at.scale = scale;
-        at.partial = partial_.as<float>(); at.partial_capacity = int(partial_.bytes / sizeof(float));
+        const DeviceBuffer& partial = M > 1 ? rows_partial_ : partial_;
+        at.partial = partial.as<float>(); at.partial_capacity = int(partial.bytes / sizeof(float));
         at.counters = counters_.as<unsigned>();
         at.position_ptr = position_ptr;
         at.spans = spans;

@@ -209,3 +209,17 @@ def test_few_keys(rt, tokens, position, heads, kv, dim, window):
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.isnan(want).any()
     plain = np.isfinite(want)
     assert np.max(np.abs(got[plain] - want[plain])) <= 2.0 ** -24 * 40 * np.nanmax(np.abs(values))
+
+
+def test_decoder_prompt_in_chunks(rt, oracle, artifacts):
+    # a decoder's chunks behind cached keys, which share those keys out over
+    # blocks: every row of logits against the CPU path (1e-3 of the largest, as
+    # for any FP32-math decoder)
+    dec, cpu = rt.Decoder(artifacts["qwen"], max_prefill=512), oracle.decoder(artifacts["qwen"], 32, False)
+    prompt = np.random.default_rng(5).integers(0, dec.vocabulary_size, 900).astype(np.uint32)
+    start = 0
+    for tokens in (512, 300, 60, 16, 10, 2):
+        ids = prompt[start:start + tokens]
+        got, want = dec.forward(ids, all_logits=True), cpu.forward(ids, all_logits=True)
+        assert np.max(np.abs(got - want)) <= 1e-3 * np.max(np.abs(want))
+        start += tokens

@@ -113,3 +113,54 @@ def test_unaligned_quantized_input(fake_hip):  # noqa: F811
         assert len(captured) == 1 and "gemm_grouped_kernel" in captured[0] and "Lb0E" in captured[0]
     status, launched = result[2]
     assert status == 0 and len(launched) == 1 and "Lb0E" in launched[0]
+
+
+PRESETS = {"qwen": (14, 2, 64), "smollm2": (15, 5, 64), "heads of 128": (32, 8, 128)}
+
+
+@pytest.mark.parametrize("shape", PRESETS)
+def test_prompts_share_their_keys_as_layer_calls_do(fake_hip, shape, tmp_path):  # noqa: F811
+    # a session's scratch is enough for every prompt length and position: its
+    # attention launches the grids of the layer call, which allocates what it needs
+    heads, kv, dim = PRESETS[shape]
+    wrong, split = fake_hip(f"""
+        from dataclasses import replace
+        from leaf_amd import artifact, models
+        spec = models.PRESETS["smollm2"](reduced=True)
+        spec = replace(spec, hidden={heads * dim}, layers=1, heads={heads}, kv_heads={kv}, head_dim={dim}, max_positions=4096)
+        path = sys.argv[2] + "/one.leaf"
+        artifact.write_artifact(path, spec, seed=1)
+        decoder = rt.Decoder(path, 32, max_context=4096, max_prefill=512)
+        def grids(): return [e[2:3] + e[4:] for e in log() if e[0] == "launch" and "attention" in e[2]]
+        wrong, split = [], 0
+        for tokens in (2, 3, 5, 16, 33, 64, 100, 191, 256, 400, 511, 512):
+            for position in (0, 1, 63, 150, 700, 1500, 2500, 3584):
+                decoder.reset()
+                done = 0
+                while done < position:
+                    n = min(512, position - done)
+                    decoder.forward_into(np.zeros(n, np.uint32), None)
+                    done += n
+                log()
+                decoder.forward_into(np.zeros(tokens, np.uint32), None)
+                session = grids()
+                assert attention(tokens, position, {heads}, {kv}, {dim}) == 0
+                if session != grids(): wrong.append([tokens, position])
+                split += len(session) == 2
+        result = wrong, split
+    """, str(tmp_path))
+    assert wrong == [] and split >= 40
+
+
+def test_session_without_memory_for_partial_results(fake_hip, tmp_path):  # noqa: F811
+    launched = fake_hip("""
+        from leaf_amd import artifact, models
+        path = sys.argv[2] + "/tiny.leaf"
+        artifact.write_artifact(path, models.PRESETS["qwen"](reduced=True), seed=1)
+        fake.fake_set_malloc_limit(5 << 20)              # the model and its workspaces fit, 9 MB of partial results do not
+        decoder = rt.Decoder(path, 32, max_context=512, max_prefill=256)
+        log()
+        decoder.forward_into(np.zeros(200, np.uint32), None)
+        result = [k for k in kernels() if "attention" in k]
+    """, str(tmp_path))
+    assert len(launched) == 2 and all("attention_rows_kernel" in k for k in launched)    # one a layer
