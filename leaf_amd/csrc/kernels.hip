@@ -113,7 +113,8 @@ __global__ __launch_bounds__(kWideRow) void norm_kernel(const float* x, int widt
 // 1024 threads: element 64 w + l of each 1024 is lane l of wave w there, each
 // wave's sum the same butterfly, the waves' sums added in order (waves past
 // the row add zeros, which change nothing), so the outputs are the same bits.
-// 2048 rows of 960: 7.2 us (12.1 as a block of sixteen waves per row).
+// 2048 rows of 960: 6.9 us (11.3 as a block of sixteen waves per row), 9.8 of a
+// trace's kernel time where the rows come from HBM.
 template <int V>
 __global__ __launch_bounds__(kBlock) void norm_wave_rows_kernel(const float* x, int rows, int width, NormView norm, float* y,
                                                                 int rows_per_group, size_t group_stride) {
@@ -1753,9 +1754,10 @@ void launch_embedding(const WeightView& table, const WeightView* positions, cons
 void launch_norm(const float* x, int rows, int width, const NormView& norm, float* y, hipStream_t stream,
                  int rows_per_group, size_t group_stride) {
     // rows enough to fill the CUs with a wave each; fewer take sixteen waves
-    // each, for the latency of one row (512 rows of 960: 4.3 against 5.5 us, 777
-    // of 896: 6.3 against 5.4)
-    if (rows >= 768 && width <= 2048 && !(norm.kind == 0 && norm.accurate)) {
+    // each, for the latency of one row (a wave per row against sixteen, in us:
+    // 768 rows of 960 5.4 and 5.5, 512 of 960 5.5 and 4.3; 1000 rows of 2048 9.0
+    // and 7.5, 1500 of 2048 10.6 and 10.2, 1600 of 2048 10.7 and 11.5)
+    if (rows >= (width <= 1024 ? 768 : 1536) && width <= 2048 && !(norm.kind == 0 && norm.accurate)) {
         const int grid = ceil_div(rows, kBlock / kWave), values = ceil_div(width, kWave);
 #define LEAF_ROWS(V) norm_wave_rows_kernel<V><<<grid, kBlock, 0, stream>>>(x, rows, width, norm, y, rows_per_group, group_stride)
         if (values <= 2) LEAF_ROWS(2);

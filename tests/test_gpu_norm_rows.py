@@ -8,7 +8,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("width", [1, 64, 77, 128, 500, 960, 1024, 1025, 2048])
-@pytest.mark.parametrize("rows", [768, 1031])
+@pytest.mark.parametrize("rows", [768, 1031, 1536])
 def test_many_rows_equal_few(width, rows):
     from leaf_amd import runtime as rt
     rng = np.random.default_rng(width + rows)

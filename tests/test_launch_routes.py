@@ -28,3 +28,14 @@ def test_attention_over_few_keys(fake_hip, heads, kv, dim, tokens, position, sma
         result = kernels()
     """)
     assert len(launched) == 1 and (f"16attention_kernelILi{1 if dim > 32 else 2}E" if small else "attention_rows_kernel") in launched[0]
+
+
+@pytest.mark.parametrize("rows,width,waves", [(767, 960, False), (768, 1024, True), (1000, 2048, False), (1535, 1025, False),
+                                              (1536, 2048, True), (4096, 2049, False)])
+def test_norm_rows(fake_hip, rows, width, waves):  # noqa: F811
+    # a wave per row only where that is the faster one
+    launched = fake_hip(f"""
+        rt.check(lib.lh_rmsnorm(buffer.ptr, {rows}, {width}, buffer.ptr, 1e-5, 0, buffer.ptr, None))
+        result = kernels()
+    """)
+    assert len(launched) == 1 and ("norm_wave_rows_kernel" in launched[0]) == waves
