@@ -19,7 +19,7 @@
 // The matrix core rounds once per product of 32 K values, so the sums lose
 // less than a chain of f32 multiply-adds does.  A value whose pieces are not
 // finite (infinity, NaN, or a magnitude that rounds past bf16's largest) gives
-// a non-finite sum; such outputs are recomputed as a plain f32 chain.
+// a non-finite sum; such outputs are recomputed in plain f32.
 //
 // Fragments.  v_mfma_f32_16x16x32_bf16: the weight rows are its A operand and
 // the tokens its B operand, lane l supplying row (token) l % 16 and the K
@@ -257,25 +257,48 @@ __device__ __forceinline__ void unit_planes(const RawUnit<BITS>& u, float scale0
 
 __device__ __forceinline__ bool finite(float v) { return __builtin_fabsf(v) < INFINITY; }
 
-// One output as a chain of f32 multiply-adds: where the split sum is not finite.
+// The lane's number, from no register that would stay live for it (one or two
+// more and some of the kernels below lose a wave per SIMD).
+__device__ __forceinline__ int this_lane() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0)); }
+
+// Where the split sum is not finite: outputs t, row..row + 3 in f32, by the whole
+// wave (rows past the last give the last one's).  One infinite activation
+// spoils its token's every output: 300 tokens x 5120 BF16 rows x 960 with one
+// such token take 62 us, with 300 735 (19 without; 2,612 and 3,558 as one
+// chain per lane).
 template <int BITS>
-__device__ __forceinline__ float plain_dot(const WeightView& w, const float* x, int t, int n) {
+__device__ __forceinline__ void plain_quad(const WeightView& w, const float* x, int t, int row, float (&sum)[4]) {
     const int K = w.cols, groups = BITS <= 8 ? K / w.group : 1;
-    float sum = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) sum[r] = 0.0f;
 #pragma unroll 1
-    for (int k = 0; k < K; ++k) {
-        const size_t at = (size_t)n * K + k;
-        float v;
-        if constexpr (BITS == 32) v = ((const float*)w.data)[at];
-        else if constexpr (BITS == 16) v = bf16_to_f32(((const uint16_t*)w.data)[at]);
-        else {
-            const int q = BITS == 8 ? (int)((const int8_t*)w.data)[at] : nibble(((const uint8_t*)w.data)[at / 2], at & 1);
-            v = (float)q * w.scales[(size_t)n * groups + k / w.group];
+    for (int k = 4 * this_lane(); k < K; k += 256) {
+        const v4f xv = *(const v4f*)(x + (size_t)t * K + k);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int n = min(row + r, w.rows - 1);
+            const uint8_t* p = (const uint8_t*)w.data + ((size_t)n * K + k) * BITS / 8;
+            float v[4];
+            if constexpr (BITS == 32) {
+                const v4f u = *(const v4f*)p;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = u[e];
+            } else if constexpr (BITS == 16) {
+                const v2u u = *(const v2u*)p;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = bf16_to_f32((u[e / 2] >> (16 * (e & 1))) & 0xFFFFu);
+            } else {
+                const float scale = w.scales[(size_t)n * groups + k / w.group];   // groups are whole quads
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    v[e] = (float)(BITS == 8 ? (int)(int8_t)p[e] : nibble(p[e / 2], e & 1)) * scale;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum[r] = fmaf(xv[e], v[e], sum[r]);
         }
-        sum = fmaf(x[(size_t)t * K + k], v, sum);
-        if (sum != sum) break;      // stays NaN
     }
-    return sum;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) sum[r] = wave_sum_f32(sum[r]);
 }
 
 // The operand planes of product q of a 16 x 16 x 32 step, small products first.
@@ -481,16 +504,18 @@ __global__ __launch_bounds__(64 * WM, 2) void gemm_f32_tiled_kernel(WeightView w
             }
         }
     }
-    while (bad) {
-        const int b = __builtin_ctz(bad);
-        bad &= bad - 1;
-        const int t = m0 + 16 * (b / NT) + li;
-#pragma unroll 1
-        for (int r = 0; r < 4; ++r) {
-            const int row = n0 + 16 * (b % NT) + 4 * lq + r;
-            if (row >= N) continue;
-            float* out = y + (size_t)t * N + row;
-            const float v = plain_dot<BITS>(w, x, t, row) + (w.bias ? w.bias[row] : 0.0f);
+    // the wave's lanes bring their quads up one after the other
+    while (const uint64_t lanes = __ballot(bad != 0)) {
+        const int from = __builtin_ctzll(lanes), b = __builtin_ctz((uint32_t)__shfl((int)bad, from, 64));
+        const int lane = this_lane();
+        if (lane == from) bad &= bad - 1;
+        const int t = m0 + 16 * (b / NT) + (from & 15), row = n0 + 16 * (b % NT) + 4 * (from >> 4);
+        float sum[4];
+        plain_quad<BITS>(w, x, t, row, sum);
+        if (lane < 4 && row + lane < N) {
+            float* out = y + (size_t)t * N + row + lane;
+            const float v = (lane & 2 ? lane & 1 ? sum[3] : sum[2] : lane & 1 ? sum[1] : sum[0]) +
+                            (w.bias ? w.bias[row + lane] : 0.0f);
             *out = epilogue == kAccumulate ? *out + v : v;
         }
     }
@@ -597,12 +622,21 @@ __global__ __launch_bounds__(64 * WK) void gemm_f32_few_kernel(WeightView w, con
         const int i = tok / 16, n = col / 16;
         const int at = (i * NT + n) * 256 + 4 * (16 * ((tok & 15) >> 2) + (col & 15)) + (tok & 3);
         const int t = m0 + tok, row = n0 + col;
-        if (t >= tokens || row >= N) continue;
+        const bool live = t < tokens && row < N;
         float v = 0.0f;
 #pragma unroll
         for (int q = 0; q < WK; ++q) v += red[q * kWaveFloats + at];
-        if constexpr (MODE == kExactRow && BITS <= 8) v *= w.scales[row] * kScaleFactor<BITS>;
-        if (!finite(v)) v = plain_dot<BITS>(w, x, t, row);
+        if constexpr (MODE == kExactRow && BITS <= 8) v *= w.scales[min(row, N - 1)] * kScaleFactor<BITS>;
+        // (four lanes in a row have one token and four rows of weights)
+        for (uint64_t lanes = __ballot(live && !finite(v)); lanes;) {
+            const int from = __builtin_ctzll(lanes) & ~3;
+            lanes &= ~((uint64_t)15 << from);
+            float sum[4];
+            plain_quad<BITS>(w, x, __shfl(t, from, 64), __shfl(row, from, 64), sum);
+            if ((lane & ~3) == from && !finite(v))
+                v = lane & 2 ? lane & 1 ? sum[3] : sum[2] : lane & 1 ? sum[1] : sum[0];
+        }
+        if (!live) continue;
         v += w.bias ? w.bias[row] : 0.0f;
         float* out = y + (size_t)t * N + row;
         *out = epilogue == kAccumulate ? *out + v : v;

@@ -112,3 +112,32 @@ def test_values_that_do_not_split(rt, bits, K, M, N):
         assert np.array_equal(np.isinf(y), np.isinf(e)) and np.array_equal(np.sign(y[np.isinf(y)]), np.sign(e[np.isinf(e)]))
         plain = np.isfinite(e)
         assert np.all(np.abs(y - e)[plain] <= 1e-4 * (1 + np.abs(e[plain])))
+
+
+@pytest.mark.parametrize("bits,M", [(32, 300), (16, 300), (4, 300), (16, 16)])
+def test_one_infinite_activation_costs_little(rt, bits, M):
+    # The outputs it spoils are computed again, by whole waves: 3 to 6 times the
+    # call's time as they are spread here (over 50 times as one chain per lane).
+    import ctypes as C
+    rng = np.random.default_rng(3)
+    K, N = 960, 5120
+    data, scales, group, _ = weights(rng, bits, N, K, 32 if bits == 4 else 0)
+    dw = rt.DeviceWeight(data, bits, K, scales, group)
+    x = rng.standard_normal((M, K), dtype=np.float32)
+    dy, lib = rt.DeviceArray((M, N), np.float32), rt.library()
+
+    def milliseconds(dx):
+        best = np.inf
+        for _ in range(5):
+            timer, ms = C.c_void_p(), C.c_double()
+            rt.linear(dw, dx, M, 32, dy)
+            rt.check(lib.lh_timer_start(None, C.byref(timer)))
+            for _ in range(5):
+                rt.linear(dw, dx, M, 32, dy)
+            rt.check(lib.lh_timer_stop(timer, None, C.byref(ms)))
+            best = min(best, ms.value)
+        return best
+
+    plain = milliseconds(rt.DeviceArray.of(x))
+    x[M // 2, K // 3] = np.inf
+    assert milliseconds(rt.DeviceArray.of(x)) <= 12 * plain
