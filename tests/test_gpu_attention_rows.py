@@ -223,3 +223,35 @@ def test_decoder_prompt_in_chunks(rt, oracle, artifacts):
         got, want = dec.forward(ids, all_logits=True), cpu.forward(ids, all_logits=True)
         assert np.max(np.abs(got - want)) <= 1e-3 * np.max(np.abs(want))
         start += tokens
+
+
+@pytest.mark.parametrize("every", [False, True])
+def test_nan_queries_cost_little(rt, every):
+    # Their rows are computed again, which ends at the first NaN score: about 1.1
+    # times the call's time for one, 7 times for all (3 and over 90 in two passes).
+    import ctypes as C
+    rng = np.random.default_rng(2)
+    heads, kv, dim, tokens = 14, 2, 64, 300
+    q, keys, values = inputs(rng, tokens, 0, heads, kv, dim)
+    dk, dv, out, lib = rt.DeviceArray.of(keys), rt.DeviceArray.of(values), rt.DeviceArray((tokens, heads, dim), np.float32), rt.library()
+
+    def milliseconds(q):
+        dq, best = rt.DeviceArray.of(q), np.inf
+        for _ in range(5):
+            timer, ms = C.c_void_p(), C.c_double()
+            for timed in (False, True):
+                if timed:
+                    rt.check(lib.lh_timer_start(None, C.byref(timer)))
+                for _ in range(5):
+                    rt.check(lib.lh_attention(dq.ptr, dk.ptr, dv.ptr, keys.shape[1], heads, kv, dim, tokens, 0, 0, out.ptr, None))
+            rt.check(lib.lh_timer_stop(timer, None, C.byref(ms)))
+            best = min(best, ms.value)
+        return best
+
+    plain = milliseconds(q)
+    spoilt = q.copy()
+    if every:
+        spoilt[:, :, 1] = np.nan
+    else:
+        spoilt[0, tokens // 2, 1] = np.nan
+    assert milliseconds(spoilt) <= (25 if every else 2) * plain
