@@ -682,12 +682,14 @@ constexpr double kCost[3][kShapes][4] = {
      {2.72, 0, 0.00197, 0.154}, {2.4, 0.000155, 0.00318, 0}, {2.39, 0.000136, 0.00342, 0},
      {2.61, 0.000128, 0.00473, 0.595}, {2.05, 0, 0.00751, 3.79}}};
 
-// LEAF_F32_GEMM_TILE=128x64|64x128|128x128|64x64 (tokens x rows) forces a tile
-// (tests compare them); any other value, or none, lets the cost decide.
+// LEAF_F32_GEMM_TILE=128x64|64x128|128x128|64x64|few16x16|few32x16|few16x32|
+// few32x32|few64x32 (tokens x rows) forces a block (tests compare them); any
+// other value, or none, lets the cost decide.
 Shape choose_shape(int mode, int tokens, int rows, int K) {
     if (const char* v = getenv("LEAF_F32_GEMM_TILE")) {
-        const char* names[] = {"128x64", "64x128", "128x128", "64x64"};
-        for (int i = 0; i < 4; ++i)
+        const char* names[kShapes] = {"128x64",   "64x128",   "128x128",  "64x64",   "few16x16",
+                                      "few32x16", "few16x32", "few32x32", "few64x32"};
+        for (int i = 0; i < kShapes; ++i)
             if (strcmp(v, names[i]) == 0) return Shape(i);
     }
     Shape best = k128x64;
