@@ -71,6 +71,7 @@ sys.path.insert(0, str(ROOT))
 HBM_PEAK_GBS = 8000.0          # MI355X HBM3E, datasheet
 INT8_PEAK_TOPS = 5000.0        # MI355X dense int8 MFMA, datasheet
 F32_PEAK_TFLOPS = 157.3        # MI355X dense f32 MFMA, datasheet
+BF16_PEAK_TFLOPS = 2500.0      # MI355X dense bf16 MFMA, datasheet
 TRAFFIC_FILE = ROOT / "profiles" / "decode_step_tinyllama_w8a8_traffic.json"
 COPY_BYTES = 1 << 30           # hbm_copy 1024: reads and writes this many bytes per launch
 GOLDEN = ROOT / "tests" / "golden"
@@ -354,6 +355,7 @@ def config_benchmark(family: str, profile_steps: int = 32) -> dict:
     steps and of the prefill for algorithmic bytes, operations and device time
     per kernel class."""
     from leaf_amd import runtime
+    from leaf_amd.models import PRESETS
     meta_all, arrays = golden()
     m = meta_all[family]
     path = ensure_artifact(family)
@@ -400,6 +402,8 @@ def config_benchmark(family: str, profile_steps: int = 32) -> dict:
     gemm = {k: v for k, v in prefill_profile.items() if k.startswith("gemm")}
     gemm_ms = sum(v["ms"] for v in gemm.values())
     gemm_tflops = sum(v["ops"] for v in gemm.values()) / max(gemm_ms, 1e-9) / 1e9
+    spec = PRESETS[family]()
+    products = 6 if spec.bits == 32 and not spec.source_bf16 else 3      # gemm_f32.hip: FP32 weights are split too
     reference = arrays[f"{family}_tokens"].tolist()
     return {
         "workload": f"{family}: {m['prompt_tokens']}-token prompt + {m['generate']} greedy tokens, "
@@ -407,8 +411,8 @@ def config_benchmark(family: str, profile_steps: int = 32) -> dict:
         "prefill_ms": round(cold_ms, 2), "prefill_warm_p50_ms": round(prefill_ms, 3),
         "prefill_TFLOPs": round(flops / prefill_ms / 1e9, 2),
         "prefill_gemm": {"ms": round(gemm_ms, 3), "TFLOPs": round(gemm_tflops, 2),
-                         # of the f32 matrix instruction's rate; the GEMM splits f32 into bf16 products and passes 1
-                         "frac_f32_mfma": round(gemm_tflops / F32_PEAK_TFLOPS, 4)},
+                         # of the bf16 matrix cores, for the products that a product of two values takes
+                         "bf16_products": products, "frac_bf16_mfma": round(gemm_tflops * products / BF16_PEAK_TFLOPS, 4)},
         "decode_tok_s": round(1e3 / decode_ms, 1), "decode_p50_ms": round(float(np.median(step_ms)), 4),
         "decode_mean_ms": round(decode_ms, 4), "bytes_per_token": round(bytes_per_token),
         "decode_GBps": round(bytes_per_token / decode_ms / 1e6, 1),
@@ -422,7 +426,7 @@ def config_benchmark(family: str, profile_steps: int = 32) -> dict:
 
 def measured_peaks() -> dict:
     """Streaming bandwidth and MFMA rates measured on this device."""
-    out = {"datasheet": {"hbm_GBps": HBM_PEAK_GBS, "int8_mfma_TOPS": INT8_PEAK_TOPS, "bf16_mfma_TFLOPs": 2500.0,
+    out = {"datasheet": {"hbm_GBps": HBM_PEAK_GBS, "int8_mfma_TOPS": INT8_PEAK_TOPS, "bf16_mfma_TFLOPs": BF16_PEAK_TFLOPS,
                          "f32_mfma_TFLOPs": F32_PEAK_TFLOPS}}
     copy = ROOT / "leaf_amd" / "bin" / "hbm_copy"
     mfma = ROOT / "leaf_amd" / "bin" / "mfma_peak"

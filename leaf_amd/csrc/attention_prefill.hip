@@ -1,15 +1,16 @@
 // Attention of several tokens (prefill, or a chunk behind cached keys) on the
 // bf16 matrix cores, with f32 accuracy.
 //
-// Every f32 operand is the exact sum of three bf16 values (split8,
-// split_bf16.h), and a product of two of them six MFMA products (those below
-// 2^-26 of it are left out), summed in f32: 2.7 times the rate of the f32
+// Every f32 operand is the sum of three bf16 values (split8, split_bf16.h),
+// exact from 2^-110 up, and a product of two of them six MFMA products (those
+// left out are at most 2^-24 of it together), summed in f32: 2.7 times the rate of the f32
 // matrix instruction, whose head-64 kernel this replaces, and any head
 // dimension up to 128.
 //
-// Rows.  The query heads of a KV head share its keys, so a block takes 64 rows
-// of one KV head, numbered token-major (row = token * group + head): a short
-// key range for causal rows, K and V split once for all of them.  Wave (wq, ws)
+// Rows.  The query heads of a KV head share its keys, so a block takes 128 rows
+// of one KV head (64 beyond head dims of 64), numbered token-major (row = token *
+// group + head): a short key range for causal rows, K and V split once for all of
+// them.  Wave (wq, ws)
 // owns 16 or 32 rows and every second 32-key slice (ws), each with its own
 // online softmax; the slices merge at the end.
 //
@@ -22,11 +23,12 @@
 // A row whose result is not finite (infinities, NaN, values past bf16's
 // range) is computed again with plain f32 arithmetic.
 //
-// What bounds it: vector instructions (softmax, splitting P, K and V), then
-// MFMAs, which
-// the barriers of a step keep from overlapping much.  2048 tokens of 14 heads of
-// 64 over 2 KV heads take 81 us (124 with f32 MFMAs), 256 tokens of 32 heads of
-// 128 behind 1000 keys 54 us (905 in a kernel without MFMAs).
+// What bounds it: vector instructions (softmax, splitting P, K and V), which
+// issue for 60% of a busy CU's time at heads of 64 and 53% at heads of 128, then
+// MFMAs (34% and 31%), which the barriers of a step keep from overlapping much.
+// 2048 tokens of 14 heads of 64 over 2 KV heads take 83 us and 10 for the merge
+// (124 with f32 MFMAs), 256 tokens of 32 heads of 128 behind 1000 keys 48 and 5
+// (905 in a kernel without MFMAs).
 #include <algorithm>
 #include <cstdint>
 #include <type_traits>

@@ -6,18 +6,19 @@
 // (decoder.cpp:236-251's storage).
 //
 // Why bf16.  The f32 matrix instruction runs at 1/15 of the bf16 one's rate
-// (156 against 2255 TFLOP/s measured on this card), and an f32 value is the
-// sum of three bf16 values without loss: hi = rn(x), mid = rn(x - hi),
-// lo = x - hi - mid (both differences are exact, and 24 significant bits are
-// three times eight).  A product of two bf16 values is exact in f32, so
+// (156 against 2255 TFLOP/s measured on this card), and an f32 value from 2^-110
+// up is the sum of three bf16 values: hi = rn(x), mid = rn(x - hi),
+// lo = x - hi - mid (split_bf16.h).  A product of two bf16 values is exact in f32, so
 //   BF16 weights:  x w = hi w + mid w + lo w                3 MFMA products;
 //   int8 / int4:   the integer is a bf16 value, the products are summed per
 //                  scale group and the group's sum enters with one fused
 //                  multiply-add of its scale                3 products;
-//   f32 weights:   w is split as well; the products below 2^-26 of x w
-//                  (mid lo, lo mid, lo lo) are left out    6 products.
+//   f32 weights:   w is split as well; mid lo, lo mid and lo lo are left out
+//                  (at most 2^-24 of x w together, 1e-8 rms)   6 products.
 // The matrix core rounds once per product of 32 K values, so the sums lose
-// less than a chain of f32 multiply-adds does.  A value whose pieces are not
+// less than a chain of f32 multiply-adds does (over 960 columns 1.0e-7 of the
+// result for BF16 weights and 1.2e-7 for f32 ones, against 5.6e-7 with the f32
+// matrix instruction).  A value whose pieces are not
 // finite (infinity, NaN, or a magnitude that rounds past bf16's largest) gives
 // a non-finite sum; such outputs are recomputed in plain f32.
 //
@@ -325,10 +326,13 @@ constexpr int x_plane(int q) {
 // (conditional loads made every wait a full one: 100 instead of 66 us for 777
 // tokens x 896 rows x 4864).
 //
-// What bounds it: 2048 tokens x 5120 BF16 rows x 960 takes 68 us (was 221 with
+// What bounds it: 2048 tokens x 5120 BF16 rows x 960 takes 67 us (was 221 with
 // f32 MFMAs): 30 us of MFMAs at the rate the card holds on such data (2.0
 // PFLOP/s at 2.06 GHz), 8 us to write the 42 MB result, the rest the staging of
-// a stage and the last, partly filled round of blocks.  Splitting x
+// a stage and the last, partly filled round of blocks.  While a CU is busy its
+// matrix cores are for 50% of the time and vector instructions issue for 49%.
+// Where the tiles are few (the same block's down projection, 960 rows x 2560:
+// 256 blocks, one wave a SIMD) 30% and 27%: loads are waited for.  Splitting x
 // in a pass of its own measured the same (68 us, 5 of them the pass).
 template <int BITS, int MODE, bool TAIL, int MT, int NT, int WM>
 __global__ __launch_bounds__(64 * WM, 2) void gemm_f32_tiled_kernel(WeightView w, const float* __restrict__ x, int tokens,
@@ -526,7 +530,10 @@ __global__ __launch_bounds__(64 * WM, 2) void gemm_f32_tiled_kernel(WeightView w
 // still keeps enough loads in flight on enough CUs.  Each wave moves both
 // operands through LDS of its own (each weight is used by one wave only); the
 // waves' sums are added in wave order.  Bound by the latency of ns / WK stages:
-// 16 tokens x 768 f32 rows x 3072 take 7.8 us (was 64 as 12 blocks of 64 x 64).
+// 16 tokens x 768 f32 rows x 3072 take 7.8 us (was 64 as 12 blocks of 64 x 64);
+// where blocks are many by splitting x, once for every 32 weight rows (777
+// tokens x 896 INT4 rows x 4864, 67 us: vector instructions issue for 69% of a
+// CU's time, MFMAs run for 21%).
 template <int BITS, int MODE, bool TAIL, int MT, int NT, int WK>
 __global__ __launch_bounds__(64 * WK) void gemm_f32_few_kernel(WeightView w, const float* __restrict__ x, int tokens,
                                                                  float* __restrict__ y, int epilogue) {

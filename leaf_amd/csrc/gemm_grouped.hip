@@ -5,8 +5,8 @@
 // for int8 or int4 weights whose groups are whole multiples of 32 values, one
 // group per row included (decoder.cpp:571-627, 661-702).  A group's integer sum
 // is exact; its term enters with the CPU path's roundings, groups in ascending
-// order, so every output is bit-identical to it.  That order is a chain, so K
-// is not split.
+// order, so every output is bit-identical to it.  One wave forms an output's sums
+// and adds its terms as they come: K is not split.
 //
 // v_mfma_i32_16x16x32_i8: the tokens are the A operand and the weight rows the
 // B operand, so a lane holds four tokens of one weight row (one weight scale
@@ -21,12 +21,15 @@
 // 128 values a stage, three or four stages ahead; rows of 128 (int4 weights 64) bytes hold segment
 // c in slot c ^ (r % 8) (c ^ (r / 2 % 4)), as in gemm_w8a8.hip.
 //
-// What bounds it: three vector instructions per output and group (convert,
-// multiply, multiply-add), three times the MFMA's cycles at 32-value groups, and
-// for short inputs the chain of stages.  Small tiles keep them on all CUs: 201 tokens x 4864 INT4 rows x 896 in
-// groups of 32 take 17 us (3,420 as one thread per output), 96 tokens x
-// 2048 x 2048 INT8 in groups of 128 13 us (56 with operands loaded where
-// they were used), 5 of each the quantization.
+// What bounds it.  Groups of 32 (201 tokens x 4864 INT4 rows x 896, 17 us, 3,440
+// as one thread per output): vector instructions issue for 75% of a busy CU's
+// time, MFMAs run for 8%.  They are ten for 64 outputs and a group, three of them
+// the term's (convert, multiply, multiply-add), the rest clearing the sums, int4
+// operands and addresses; and of 1064 blocks 1024 are resident at once (35 KB of
+// LDS each).  Long groups over few blocks (96 tokens x 2048 x 2048 INT8 in groups
+// of 128, 12 us, 56 with operands loaded where they were used): the latency of a
+// block's 16 stages, vector instructions at 22%, waits for half the time.  About 4
+// us of either are the quantization.
 #include <type_traits>
 
 #include "device_common.h"
