@@ -141,7 +141,12 @@ public:
     // this one's calls), on the per-thread default stream, whose one handle
     // stands for a stream of each thread, and where the device has no memory left.
     void* work_if_own(size_t bytes) {
-        if (stream_ == hipStreamPerThread || capturing(stream_)) return nullptr;
+        try {
+            if (stream_ == hipStreamPerThread || capturing(stream_)) return nullptr;
+        } catch (const leafhip::Error&) {
+            (void)hipGetLastError();   // the null stream may not be asked beside a capture
+            return nullptr;
+        }
         try {
             return work(bytes);
         } catch (const leafhip::Error& e) {

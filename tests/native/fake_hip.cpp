@@ -16,7 +16,7 @@
 
 struct dim3 { uint32_t x, y, z; };
 typedef void* stream_t;
-enum { kSuccess = 0, kOutOfMemory = 2 };
+enum { kSuccess = 0, kOutOfMemory = 2, kCaptureImplicit = 906 };
 
 static std::mutex g_lock;
 static std::string g_log;
@@ -99,7 +99,11 @@ int hipMemcpy2DAsync(void* dst, size_t dpitch, const void* src, size_t spitch, s
 }
 int hipMemset(void* p, int value, size_t bytes) { std::memset(p, value, bytes); return kSuccess; }
 int hipMemsetAsync(void* p, int value, size_t bytes, stream_t) { return hipMemset(p, value, bytes); }
-int hipStreamIsCapturing(stream_t, int* status) { *status = g_capturing ? 1 : 0; return kSuccess; }
+int hipStreamIsCapturing(stream_t stream, int* status) {
+    if (!stream && g_capturing) return t_error = kCaptureImplicit;   // the null stream, beside a capture
+    *status = g_capturing ? 1 : 0;
+    return kSuccess;
+}
 int hipGetLastError() { const int e = t_error; t_error = kSuccess; return e; }
 const char* hipGetErrorString(int) { return "fake HIP error"; }
 int hipGetDevice(int* d) { *d = 0; return kSuccess; }

@@ -60,13 +60,15 @@ def test_captured_attention_keeps_no_scratch(fake_hip):  # noqa: F811
         fake.fake_set_capturing(1)
         assert attention(64, 1000, stream=stream.handle) == 0
         captured = kernels()
+        assert attention(64, 1000) == 0              # on the null stream, which may not be asked then
+        captured += kernels()
         fake.fake_set_capturing(0)
         # one handle for every thread's own default stream
         assert attention(64, 1000, stream=2) == 0
         result = eager, captured, kernels()
     """)
     assert len(eager) == 2 and "merge" in eager[1]
-    assert len(captured) == 1 and "attention_rows_kernel" in captured[0]
+    assert len(captured) == 2 and all("attention_rows_kernel" in k for k in captured)
     assert len(per_thread) == 1 and "attention_rows_kernel" in per_thread[0]
 
 
