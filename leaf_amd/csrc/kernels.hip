@@ -16,6 +16,8 @@
 
 #include <math.h>
 
+#include <type_traits>
+
 namespace leafhip {
 namespace {
 
@@ -1099,11 +1101,11 @@ __global__ __launch_bounds__(kBlock) void rope_kv_quads_kernel(RopeKvCall p) {
 // (dot * scale) * scale; the softmax is rescaled per key block, so results
 // agree with the CPU's max / exp / sum / divide to rounding.
 // kFew...: calls over a few dozen keys that could take the matrix cores' kernel.
-// As exact as there: eight fused chains added at the end (one in
-// 64 bits up to 32 dims), the scale applied to their distance from the maximum.
-// 16 tokens behind 20 keys, relative to 64 bits, the matrix cores' kernel second:
-// 1.6e-7 against 2.3e-7 for heads of 128, 1.4e-7 and 1.7e-7 (64), 1.1e-7 both
-// (32).  (Over many keys the chains cost more than they give: 300 tokens of 8
+// As exact as there: eight fused chains added at the end (up to 32 dims one in 64
+// bits, and the outputs too), the scale applied to their distance from the
+// maximum.  16 tokens behind 62 keys, relative to 64 bits, the matrix cores'
+// kernel second: 1.9e-7 against 2.9e-7 for heads of 128, 1.7e-7 and 2.0e-7 (64),
+// 1.2e-7 and 1.4e-7 (32).  (Over many keys the chains cost more than they give: 300 tokens of 8
 // heads of 160 behind 500 keys 298 instead of 245 us.)
 // Grid: (heads, tokens, splits).  With splits > 1 (decode) each block writes
 // (max, sum, o[dim]) for its key range to `partial`, merged by attention_merge.
@@ -1133,7 +1135,7 @@ __global__ __launch_bounds__(kBlock) void attention_kernel(AttentionCall p, int 
     const float scale2 = SCORE != kSequential ? p.scale * p.scale : 1.0f;       // what scores are still to be multiplied by
     // thread owns output dims d = tid % 64 (+64, ...) for key lane kl = tid / 64
     const int dl = threadIdx.x & 63, kl = threadIdx.x >> 6;
-    float o[4] = {0.f, 0.f, 0.f, 0.f};   // dims dl, dl+64, dl+128, dl+192
+    std::conditional_t<SCORE == kFewDouble, double, float> o[4] = {};   // dims dl, dl+64, dl+128, dl+192
     for (int k0 = s_begin; k0 < s_end; k0 += kKeysPerPass) {
         const int n = min(kKeysPerPass, s_end - k0);
         float local_max = -INFINITY;
@@ -1184,7 +1186,9 @@ __global__ __launch_bounds__(kBlock) void attention_kernel(AttentionCall p, int 
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int d = dl + 64 * j;
-                if (d < dim) o[j] = fmaf(pk, vrow[d], o[j]);
+                if (d >= dim) continue;
+                if constexpr (SCORE == kFewDouble) o[j] = fma((double)pk, (double)vrow[d], o[j]);
+                else o[j] = fmaf(pk, vrow[d], o[j]);
             }
         }
         m = m_new;
@@ -1194,7 +1198,7 @@ __global__ __launch_bounds__(kBlock) void attention_kernel(AttentionCall p, int 
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int d = dl + 64 * j;
-        if (d < dim) o_s[kl][d] = o[j];
+        if (d < dim) o_s[kl][d] = (float)o[j];
     }
     __syncthreads();
     if (gridDim.z == 1) {
@@ -2013,11 +2017,16 @@ bool launch_attention(const AttentionCall& call, hipStream_t stream) {
     }
     // Over a few dozen keys one block per head and token ends before the matrix
     // cores' kernel has staged its first 64 keys (4 tokens of 32 heads of 128: 4.9
-    // against 8.7 us at once, 7.5 against 9.2 behind 32 keys).  They meet at 40 to
-    // 50 keys, for all head dims from 20 to 128 but 64, where it is later.
+    // against 8.7 us at once, 8.2 against 9.3 over 44 keys).  They meet at 48 to 56
+    // keys, for all head dims from 20 to 128 but 64, where it is later; again at
+    // 80 to 96 where the second 64 have begun (16 tokens of 8 heads of 32 over 65
+    // keys: 7.4 against 8.9).  Beyond 24 tokens of 32 heads of 128 its blocks are
+    // too many for that (48 of them over 80 keys: 1.2 times the other's time).
+    const bool light = (size_t)call.heads * call.tokens * call.dim <= 98304;
+    const bool few = total <= 40 || (light && (total <= 48 || (total > 64 && total <= 80)));
     dim3 grid(call.heads, call.tokens, splits);
     if (attention_rows_supported(call)) {
-        if (total > 40) launch_attention_rows(call, stream);
+        if (!few) launch_attention_rows(call, stream);
         else if (call.dim > 32) attention_kernel<kFewChains><<<grid, kBlock, 0, stream>>>(call, per_split);
         else attention_kernel<kFewDouble><<<grid, kBlock, 0, stream>>>(call, per_split);
         return true;

@@ -196,11 +196,12 @@ def test_general_kernel_without_a_usable_score(rt, dim, offset, spoilt):
     assert np.max(np.abs(got[plain] - want[plain])) <= 2.0 ** -24 * 40 * 5
 
 
-# Up to 40 keys (one block per head and token) and just beyond, with windows,
+# Up to 40, 48 and 80 keys (one block per head and token) and just beyond, with windows,
 # dims with and without a remainder of eight, and a NaN in between.
 @pytest.mark.parametrize("tokens,position,heads,kv,dim,window", [
     (2, 0, 12, 12, 64, 0), (40, 0, 4, 2, 128, 0), (17, 23, 6, 2, 80, 9), (5, 35, 8, 1, 32, 0), (3, 20, 4, 4, 36, 5),
-    (40, 0, 3, 3, 4, 0), (41, 0, 3, 3, 4, 0), (9, 32, 4, 2, 128, 12)])
+    (40, 0, 3, 3, 4, 0), (50, 0, 3, 3, 4, 0), (9, 32, 4, 2, 128, 12), (20, 28, 4, 2, 96, 0), (7, 60, 6, 2, 64, 0),
+    (24, 56, 32, 8, 128, 0), (25, 56, 4, 4, 32, 0), (16, 64, 8, 1, 32, 50)])
 def test_few_keys(rt, tokens, position, heads, kv, dim, window):
     rng = np.random.default_rng(tokens + dim)
     q, keys, values = inputs(rng, tokens, position, heads, kv, dim)

@@ -20,14 +20,17 @@ def test_attention_alignment(fake_hip, argument):  # noqa: F811
     assert len(unaligned) == 1 and "16attention_kernelILi0E" in unaligned[0]
 
 
-@pytest.mark.parametrize("tokens,position,small", [(2, 0, True), (4, 36, True), (40, 0, True), (2, 39, False), (41, 0, False)])
+# up to 40 keys; up to 48, and from 65 to 80, where heads, tokens and dims are few
+@pytest.mark.parametrize("tokens,position,small", [(2, 0, True), (4, 36, True), (40, 0, True), (2, 46, True), (2, 47, False),
+                                                   (4, 60, False), (4, 61, True), (16, 64, True), (16, 65, False),
+                                                   (200, 0, False)])
 @pytest.mark.parametrize("heads,kv,dim", [(32, 8, 128), (8, 1, 32), (14, 2, 64)])
 def test_attention_over_few_keys(fake_hip, heads, kv, dim, tokens, position, small):  # noqa: F811
     launched = fake_hip(f"""
         assert attention({tokens}, {position}, {heads}, {kv}, {dim}) == 0
         result = kernels()
     """)
-    assert len(launched) == 1 and (f"16attention_kernelILi{1 if dim > 32 else 2}E" if small else "attention_rows_kernel") in launched[0]
+    assert len(launched) <= 2 and (f"16attention_kernelILi{1 if dim > 32 else 2}E" if small else "attention_rows_kernel") in launched[0]
 
 
 @pytest.mark.parametrize("rows,width,waves", [(767, 960, False), (768, 1024, True), (1000, 2048, False), (1535, 1025, False),
@@ -39,3 +42,12 @@ def test_norm_rows(fake_hip, rows, width, waves):  # noqa: F811
         result = kernels()
     """)
     assert len(launched) == 1 and ("norm_wave_rows_kernel" in launched[0]) == waves
+
+
+@pytest.mark.parametrize("tokens,small", [(24, True), (25, False)])
+def test_attention_over_few_keys_of_many_heads(fake_hip, tokens, small):  # noqa: F811
+    launched = fake_hip(f"""
+        assert attention({tokens}, {72 - tokens}, 32, 8, 128) == 0
+        result = kernels()
+    """)
+    assert len(launched) == 1 and ("16attention_kernelILi1E" if small else "attention_rows_kernel") in launched[0]
