@@ -9,7 +9,7 @@
 // Decode GEMVs are HBM-bound: a wave owns whole rows, lanes stride over
 // 128-bit chunks of them (coalesced 1 KiB per wave load), and the dot product
 // is reduced across the wave with butterfly shuffles.  Prefill linears run on
-// MFMA (int8 for W8A8, f32 otherwise).
+// MFMA (int8 for integer activations, bf16 otherwise).
 #include "device_common.h"
 #include "kernels.h"
 #include "libm_expf.h"
@@ -2017,10 +2017,10 @@ bool launch_attention(const AttentionCall& call, hipStream_t stream) {
     }
     // Over a few dozen keys one block per head and token ends before the matrix
     // cores' kernel has staged its first 64 keys (4 tokens of 32 heads of 128: 4.9
-    // against 8.7 us at once, 8.2 against 9.3 over 44 keys).  They meet at 48 to 56
+    // against 8.7 us at once, 8.2 against 9.2 over 44 keys).  They meet at 48 to 56
     // keys, for all head dims from 20 to 128 but 64, where it is later; again at
     // 80 to 96 where the second 64 have begun (16 tokens of 8 heads of 32 over 65
-    // keys: 7.4 against 8.9).  Beyond 24 tokens of 32 heads of 128 its blocks are
+    // keys: 7.7 against 9.4).  Beyond 24 tokens of 32 heads of 128 its blocks are
     // too many for that (48 of them over 80 keys: 1.2 times the other's time).
     const bool light = (size_t)call.heads * call.tokens * call.dim <= 98304;
     const bool few = total <= 40 || (light && (total <= 48 || (total > 64 && total <= 80)));
